@@ -229,6 +229,8 @@ struct qs_ctx {
   // adjoint
   std::vector<DevBuf> ckpt;
   DevBuf gx, target, lossp, gT, gprobe, gV, dsum, adj_ipos;
+  DevBuf adj_order, adj_xrange;  // several probes: the reverse row sweep's work by transmission row
+  int adj_chunk = 0, adj_nchunk = 0;
   // band limit of dL/dt on the second stream: a second band-compact buffer, events
   // "row sweep wrote buffer b" and "band limit done with buffer b"
   DevBuf blstate2;
@@ -639,6 +641,7 @@ void qs_destroy(qs_ctx* c) {
                     &c->lz.tw, &c->lz.chirp_f, &c->lz.vhat_f, &c->lz.chirp_b, &c->lz.vhat_b,
                     &c->gx, &c->target, &c->lossp, &c->gT, &c->gprobe, &c->gV, &c->dsum,
                     &c->blpx, &c->blpy, &c->blstate, &c->blstate2, &c->adj_ipos,
+                    &c->adj_order, &c->adj_xrange,
                     &c->wx.tw, &c->wx.chirp_f, &c->wx.vhat_f, &c->wx.chirp_b, &c->wx.vhat_b,
                     &c->wy.tw, &c->wy.chirp_f, &c->wy.vhat_f, &c->wy.chirp_b, &c->wy.vhat_b, &c->gscratch, &c->gtiles};
   for (DevBuf* b : bufs) b->release();
@@ -2036,7 +2039,46 @@ static qs::AdjArgs adj_args(qs_ctx* c, int nprobe) {
   // every gT element is stored once per slice
   const bool whole = nprobe == 1 && p.nx == p.potNx && p.ny == p.potNy;
   A.single_writer = nprobe == 1 ? (whole ? 2 : 1) : 0;
+  A.potNx = p.potNx;
+  if (nprobe > 1) {
+    A.order = c->adj_order.as<int>();
+    A.xrange = c->adj_xrange.as<int2>();
+    A.chunk = c->adj_chunk;
+    A.nchunk = c->adj_nchunk;
+  }
   return A;
+}
+
+// Work of the reverse row sweep for several probes, by groups of transmission rows: the
+// probes in order of their x offset, of which the rows of a group are read by a contiguous
+// range; chunks of them per block.  A chunk is as long as leaves about 2048 blocks (8 per
+// CU), at most 16 probes per unit: longer chunks mean fewer additions to dL/dt in memory.
+struct AdjRowWork {
+  std::vector<int> order;
+  std::vector<int2> xrange;
+  int chunk = 1, nchunk = 1;
+};
+static AdjRowWork adj_row_work(const qs_params& p, const int* ipos, int nprobe) {
+  AdjRowWork w;
+  int group = 1, units = 1;
+  qs::adj_row_shape(p.ny, &group, &units);
+  w.order.resize(nprobe);
+  for (int i = 0; i < nprobe; i++) w.order[i] = i;
+  std::stable_sort(w.order.begin(), w.order.end(), [&](int a, int b) { return ipos[2 * a] < ipos[2 * b]; });
+  std::vector<int> x(nprobe);
+  for (int i = 0; i < nprobe; i++) x[i] = ipos[2 * w.order[i]];
+  long long pairs = 0;
+  int most = 1;
+  for (int X = 0; X < p.potNx; X += group) {
+    const int lo = (int)(std::lower_bound(x.begin(), x.end(), X - p.nx + 1) - x.begin());
+    const int hi = (int)(std::lower_bound(x.begin(), x.end(), X + group) - x.begin());
+    w.xrange.push_back(make_int2(lo, hi));
+    pairs += hi - lo;
+    most = std::max(most, hi - lo);
+  }
+  w.chunk = units * (int)std::max<long long>(1, std::min<long long>(16, pairs / (2048LL * units)));
+  w.nchunk = (most + w.chunk - 1) / w.chunk;
+  return w;
 }
 
 // First half of the adjoint: the forward pass with checkpoints (X_{jK-1} in
@@ -2087,6 +2129,14 @@ static int adj_forward(qs_ctx* c, const char* who, const int* ipos, int nprobe, 
   for (int j = 0; j < nseg + K; j++) HIPCHK(c, c->ckpt[j].ensure(st_bytes));  // [0,nseg): X_{jK-1}; [nseg,nseg+K): segment
   HIPCHK(c, c->adj_ipos.ensure(sizeof(int) * 2 * nprobe));
   HIPCHK(c, hipMemcpyAsync(c->adj_ipos.p, ipos, sizeof(int) * 2 * nprobe, hipMemcpyHostToDevice, c->stream));
+  AdjRowWork work;  // until the synchronisation below
+  if (nprobe > 1) {
+    work = adj_row_work(p, ipos, nprobe);
+    HIPCHK(c, upload(c->adj_order, work.order, c->stream));
+    HIPCHK(c, upload(c->adj_xrange, work.xrange, c->stream));
+    c->adj_chunk = work.chunk;
+    c->adj_nchunk = work.nchunk;
+  }
   const size_t nt = (size_t)nprobe * p.nx * p.ny;
   HIPCHK(c, c->target.ensure(sizeof(float) * nt));
   HIPCHK(c, hipMemcpyAsync(c->target.p, target, sizeof(float) * nt, hipMemcpyDefault, c->stream));

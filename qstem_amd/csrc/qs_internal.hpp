@@ -56,10 +56,19 @@ struct AdjArgs {
   const float2* xprev;      // forward state X_{s-1} (rows sweep, s > 0) or X_{S-1} (last column sweep)
   const float* target;      // [nprobe_total][nx][ny] target intensities, FFTW order (last column sweep)
   float* loss_partial;      // [nprobe][ntiles] (last column sweep)
-  float* gT;                // [potNx][potNy][2] gradient w.r.t. the transmission slice (atomics)
+  float* gT;                // [potNx][potNy][2] gradient w.r.t. the transmission slice
   float* gprobe;            // [nx][ny][2] sum over probes of the gradient w.r.t. psi_0 (atomics)
   int single_writer;        // 1: one probe per launch, gT updated without atomics;
-                            // 2: and its window is the whole slice, gT stored (no prior clear)
+                            // 2: and its window is the whole slice, gT stored (no prior clear);
+                            // 0: several probes (k_adj_rows_acc, the four fields below)
+  // Several probes: the launch's rows by groups of transmission rows (adj_row_shape).  Group
+  // G's rows are read by the probes order[xrange[G].x .. xrange[G].y) (order: probe indices
+  // by ascending window offset ipos.x); a block takes up to `chunk` of them, nchunk blocks
+  // per group.
+  const int* order;
+  const int2* xrange;
+  int chunk, nchunk;
+  int potNx;
   // With single_writer 2 and the transmission band limit on band-compact sweeps: the
   // row sweep stores the row FFT of each dL/dt row, band-compact in the potential
   // grid's band (bl_band_a, bl_gap, rows of bl_kcp), into blstate instead of the row
@@ -257,6 +266,8 @@ void launch_probe_window(const ProbeArgs& a, float2* psi, double* partial, hipSt
 void launch_fill_zero(float2* p, size_t n, hipStream_t st);
 hipError_t set_col_lds_limits();
 void launch_adj_rows(const AdjArgs& a, bool first_slice, hipStream_t st);
+// Several probes per launch: transmission rows per block, and probes that a block works on at once.
+void adj_row_shape(int ny, int* group, int* units);
 void launch_adj_cols(const AdjArgs& a, bool last_slice, hipStream_t st);
 void launch_grad_v(const float2* gu, const float* V, float* gV, size_t n, double sigma, hipStream_t st);
 void launch_target_outside_band(const float* target, int nprobe, int nx, int ny, int band_a, int band_b,

@@ -163,6 +163,7 @@ __global__ void k_fill_zero(float2* __restrict__ p, size_t n) {
   void rows_fft_##N(float2*, long, int, const float2*, float, hipStream_t);                         \
   void bluestein_##N(float2*, long, int, const float2*, const float2*, const float2*, float, hipStream_t); \
   void adj_rows_##N(const AdjArgs&, bool, hipStream_t);                                             \
+  void adj_row_shape_##N(int*, int*);                                                               \
   void adj_cols_##N(const AdjArgs&, bool, hipStream_t);
 QS_DECL(64)
 QS_DECL(128)
@@ -231,6 +232,12 @@ void launch_rows_bluestein(float2* d, long nrows, int n, int M, const float2* ch
 void launch_adj_rows(const AdjArgs& a, bool first_slice, hipStream_t st) {
 #define C(N) adj_rows_##N(a, first_slice, st)
   QS_SWITCH(a.f.ny, C)
+#undef C
+}
+
+void adj_row_shape(int ny, int* group, int* units) {
+#define C(N) adj_row_shape_##N(group, units)
+  QS_SWITCH(ny, C)
 #undef C
 }
 

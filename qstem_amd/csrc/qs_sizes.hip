@@ -18,6 +18,10 @@ hipError_t QS_CAT(set_col_lds_, QS_N)() {
   return e == hipSuccess ? set_adj_lds_t<QS_N>() : e;
 }
 void QS_CAT(adj_rows_, QS_N)(const AdjArgs& a, bool first, hipStream_t st) { launch_adj_rows_t<QS_N>(a, first, st); }
+void QS_CAT(adj_row_shape_, QS_N)(int* group, int* units) {
+  *group = adj_tpw<QS_N>();
+  *units = adj_units<QS_N>();
+}
 void QS_CAT(adj_cols_, QS_N)(const AdjArgs& a, bool last, hipStream_t st) { launch_adj_cols_t<QS_N>(a, last, st); }
 int QS_CAT(col_tile_, QS_N)() { return ColCfg<QS_N>::TC; }
 void QS_CAT(rows_fft_, QS_N)(float2* d, long nrows, int dir, const float2* tw, float scale, hipStream_t st) {

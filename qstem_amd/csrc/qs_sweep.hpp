@@ -782,11 +782,12 @@ __global__ __launch_bounds__(ColCfg<NX>::BLK) void k_adj_cols(AdjArgs A) {
   }
 }
 
-// Row sweep (slice s, reverse):  g_a = rowIFFT(g_R);  psi_s = rowIFFT(X_{s-1}) (or the
-// probe);  g_t += conj(psi_s) g_a;  g_psi = conj(t_s) g_a;  g_X_{s-1} = rowFFT(g_psi)
-// (s > 0) or sum_p g_psi -> gprobe (s = 0).  BLF (the window is the whole slice): the
-// row of g_t is complete here, so its row FFT, band-compact in the potential grid's
-// band, goes to A.blstate (the band limit's first pass) instead of the row to A.gT.
+// Row sweep (slice s, reverse) of a single probe:  g_a = rowIFFT(g_R);  psi_s =
+// rowIFFT(X_{s-1}) (or the probe);  g_t += conj(psi_s) g_a;  g_psi = conj(t_s) g_a;
+// g_X_{s-1} = rowFFT(g_psi) (s > 0) or g_psi -> gprobe (s = 0).  BLF (the window is the
+// whole slice): the row of g_t is complete here, so its row FFT, band-compact in the
+// potential grid's band, goes to A.blstate (the band limit's first pass) instead of the
+// row to A.gT.
 template <int NY, bool FIRST, bool BLF>
 __global__ __launch_bounds__(row_block<NY>()) void k_adj_rows(AdjArgs A) {
   const SweepArgs& a = A.f;
@@ -837,13 +838,10 @@ __global__ __launch_bounds__(row_block<NY>()) void k_adj_rows(AdjArgs A) {
       w[m] = gtv;  // kept for the row FFT below
     } else if (A.single_writer == 2) {  // the window is the whole slice: this is the pixel's only term
       *reinterpret_cast<float2*>(gt + 2 * iy) = gtv;
-    } else if (A.single_writer) {  // one probe per launch: each transmission pixel has one writer
+    } else {  // one probe per launch: each transmission pixel has one writer
       float2* p2 = reinterpret_cast<float2*>(gt + 2 * iy);
       const float2 o = *p2;
       *p2 = make_float2(o.x + gtv.x, o.y + gtv.y);
-    } else {
-      atomicAdd(gt + 2 * iy, gtv.x);
-      atomicAdd(gt + 2 * iy + 1, gtv.y);
     }
     g[m] = cmulc(g[m], tr[iy]);  // conj(t) * g_a
   }
@@ -869,8 +867,166 @@ __global__ __launch_bounds__(row_block<NY>()) void k_adj_rows(AdjArgs A) {
   }
 }
 
+// The same sweep for several probes, whose windows overlap in the slice.  A block owns a
+// group of TPW consecutive transmission rows (the rows that the transforms of one wavefront
+// work on side by side) and a chunk of the probes that read them.  Each wavefront takes a
+// contiguous run of the chunk, one probe at a time (its row bases are scalars), and sums
+// dL/dt of the rows in an LDS area of its own by plain loads and stores; at the end the
+// block adds the areas and issues one global atomic pair per touched pixel.  With one
+// global atomic pair per pixel and probe the sweep was bound by the atomics (134 M float
+// atomics per slice for 1024 probes of 256^2 in 384^2: 1346 us; with the sums as LDS float
+// atomics 1143 us; now 372 us, of which the 1.1 GB of state take 206 us at copy rate).  In the first slice a wavefront sums
+// g_psi of neighbouring probes with the same x offset in registers before the atomics on
+// gprobe.
+template <int N> constexpr int adj_tpw() { return N / Plan<N>::E <= 64 ? 64 / (N / Plan<N>::E) : 1; }
+template <int N> constexpr int adj_units() { return N / Plan<N>::E <= 64 ? row_block<N>() / 64 : 1; }
+// Widest span of a chunk's windows that is summed in LDS (48 KB per block); wider ones add
+// straight to A.gT.
+template <int N> constexpr int adj_acc_max() { return 6144 / (adj_tpw<N>() * adj_units<N>()); }
+
+template <int NY, bool FIRST>
+__global__ __launch_bounds__(row_block<NY>()) void k_adj_rows_acc(AdjArgs A) {
+  const SweepArgs& a = A.f;
+  constexpr int E = Plan<NY>::E;
+  constexpr int T = NY / E;
+  constexpr int BLK = row_block<NY>();
+  constexpr int TPW = adj_tpw<NY>();
+  constexpr int GAP = gap_mask<NY>();  // slots in the band gap: never loaded, stored or computed
+  constexpr int UPB = adj_units<NY>();  // units (wavefronts, or the block) per block
+  __shared__ float2 lds[(BLK / T) * lds_slot<NY>()];
+  __shared__ int yspan[2];
+  extern __shared__ float2 acc[];  // [UPB][TPW][span]
+  const int X0 = (blockIdx.x / A.nchunk) * TPW;
+  const int2 range = A.xrange[blockIdx.x / A.nchunk];
+  const int lo = range.x + (blockIdx.x % A.nchunk) * A.chunk, hi = min(range.y, lo + A.chunk);
+  if (lo >= hi) return;  // whole blocks
+  if (threadIdx.x == 0) {
+    yspan[0] = 0x7fffffff;
+    yspan[1] = 0;
+  }
+  __syncthreads();
+  for (int i = lo + threadIdx.x; i < hi; i += BLK) {
+    const int y = a.ipos[A.order[i]].y;
+    atomicMin(&yspan[0], y);
+    atomicMax(&yspan[1], y + NY);
+  }
+  __syncthreads();
+  const int ylo = wave_uniform(yspan[0]), span = wave_uniform(yspan[1]) - ylo;
+  const bool in_lds = span <= adj_acc_max<NY>();
+  if (in_lds) {
+    for (int i = threadIdx.x; i < UPB * TPW * span; i += BLK) acc[i] = make_float2(0.f, 0.f);
+  }
+  __syncthreads();
+  const int lane = T <= 64 ? (threadIdx.x & 63) : threadIdx.x;
+  const int unit = T <= 64 ? wave_uniform(threadIdx.x >> 6) : 0;
+  const int sub = lane / T, t = lane % T;
+  float2* slot = lds + (threadIdx.x / T) * lds_slot<NY>();
+  Twiddles<NY> tw;
+  tw.init(a.twy, t);
+  // band columns through buffer resources, as in k_adj_rows; row sub of the group at sub * rowb
+  const int gap = NY - a.band_b - a.band_a - 1;
+  const unsigned rowb = (unsigned)a.kcp * 8u;
+  unsigned bo[E];
+#pragma unroll
+  for (int m = 0; m < E; m++) {
+    const unsigned o = band_off(t + T * m, a.band_a, gap);
+    bo[m] = o == kOut ? kOut : o + (unsigned)sub * rowb;
+  }
+  const int X = X0 + sub;
+  const float2* const trow = a.trans + (size_t)min(X, A.potNx - 1) * a.potNy + t;
+  float* const grow = A.gT + 2 * ((size_t)min(X, A.potNx - 1) * a.potNy + t);
+  float2* const accr = acc + (unit * TPW + sub) * span + t;
+  const int per = (hi - lo + UPB - 1) / UPB;  // probes of this unit
+  const int i1 = min(hi, lo + (unit + 1) * per);
+  float2 gsum[FIRST ? E : 1];
+  if constexpr (FIRST) {
+#pragma unroll
+    for (int m = 0; m < E; m++) gsum[m] = make_float2(0.f, 0.f);
+  }
+  for (int i = lo + unit * per; i < i1; i++) {
+    const int p = A.order[i];
+    const int2 ip = a.ipos[p];
+    const int x0 = X0 - ip.x;  // window row of sub 0; rows outside [0, nx) read zeros and store nothing
+    const bool row = x0 + sub >= 0 && x0 + sub < a.nx;
+    const long long roff = ((long long)p * a.nx + x0) * a.kcp;
+    const rsrc_t rg = make_rsrc(A.gx + roff, (long)TPW * rowb);
+    float2 g[E], w[E];
+#pragma unroll
+    for (int m = 0; m < E; m++) g[m] = (GAP >> m) & 1 ? make_float2(0.f, 0.f) : buf_load_c64(rg, row ? bo[m] : kOut);
+    if constexpr (FIRST) {
+      const float2* pr = a.probe + (size_t)(row ? x0 + sub : 0) * NY + t;
+#pragma unroll
+      for (int m = 0; m < E; m++) w[m] = row ? pr[T * m] : make_float2(0.f, 0.f);
+    } else {
+      const rsrc_t rx = make_rsrc(A.xprev + roff, (long)TPW * rowb);
+#pragma unroll
+      for (int m = 0; m < E; m++) w[m] = (GAP >> m) & 1 ? make_float2(0.f, 0.f) : buf_load_c64(rx, row ? bo[m] : kOut);
+    }
+    fft_wave<NY, +1, kSwz<NY>, GAP>(g, slot, tw, t);
+    if constexpr (!FIRST) fft_wave<NY, +1, kSwz<NY>, GAP>(w, slot, tw, t);
+    const float2* tr = trow + ip.y;
+#pragma unroll
+    for (int m = 0; m < E; m++) {
+      const float2 gtv = cmulc(g[m], w[m]);  // conj(psi) * g_a
+      if (in_lds) {  // the unit's own area (block-wide transforms: ordered by their barriers)
+        float2* const q = accr + (ip.y - ylo) + T * m;
+        *q = cadd(*q, gtv);
+      } else if (row) {
+        atomicAdd(grow + 2 * (ip.y + T * m), gtv.x);
+        atomicAdd(grow + 2 * (ip.y + T * m) + 1, gtv.y);
+      }
+      g[m] = cmulc(g[m], tr[T * m]);  // conj(t) * g_a
+    }
+    if constexpr (FIRST) {
+#pragma unroll
+      for (int m = 0; m < E; m++) gsum[m] = cadd(gsum[m], g[m]);
+      if (i + 1 == i1 || a.ipos[A.order[i + 1]].x != ip.x) {  // the unit's next row is another row of gprobe
+        if (row) {
+          float* gp = A.gprobe + 2 * ((size_t)(x0 + sub) * NY + t);
+#pragma unroll
+          for (int m = 0; m < E; m++) {
+            atomicAdd(gp + 2 * T * m, gsum[m].x);
+            atomicAdd(gp + 2 * T * m + 1, gsum[m].y);
+          }
+        }
+#pragma unroll
+        for (int m = 0; m < E; m++) gsum[m] = make_float2(0.f, 0.f);
+      }
+    } else {
+      fft_wave<NY, -1, kSwz<NY>, 0, ~GAP>(g, slot, tw, t);
+#pragma unroll
+      for (int m = 0; m < E; m++)
+        if (!((GAP >> m) & 1)) buf_store_c64(g[m], rg, row ? bo[m] : kOut);
+    }
+  }
+  __syncthreads();
+  if (in_lds) {
+#pragma unroll 1
+    for (int r = 0; r < TPW && X0 + r < A.potNx; r++) {
+      float* const gr = A.gT + 2 * ((size_t)(X0 + r) * a.potNy + ylo);
+      for (int i = threadIdx.x; i < span; i += BLK) {
+        float2 sum = acc[r * span + i];
+#pragma unroll
+        for (int u = 1; u < UPB; u++) sum = cadd(sum, acc[(u * TPW + r) * span + i]);
+        atomicAdd(gr + 2 * i, sum.x);
+        atomicAdd(gr + 2 * i + 1, sum.y);
+      }
+    }
+  }
+}
+
+template <int N>
+void launch_adj_rows_acc_t(const AdjArgs& a, bool first, hipStream_t st) {
+  constexpr int TPW = adj_tpw<N>();
+  const dim3 grid((unsigned)((a.potNx + TPW - 1) / TPW * a.nchunk));  // adj_row_shape's rows per group
+  const size_t lds = sizeof(float2) * TPW * adj_units<N>() * (a.f.potNy < adj_acc_max<N>() ? a.f.potNy : adj_acc_max<N>());
+  if (first) hipLaunchKernelGGL((k_adj_rows_acc<N, true>), grid, dim3(row_block<N>()), lds, st, a);
+  else hipLaunchKernelGGL((k_adj_rows_acc<N, false>), grid, dim3(row_block<N>()), lds, st, a);
+}
+
 template <int N>
 void launch_adj_rows_t(const AdjArgs& a, bool first, hipStream_t st) {
+  if (!a.single_writer) return launch_adj_rows_acc_t<N>(a, first, st);
   constexpr int T = N / Plan<N>::E;
   constexpr int RPB = row_block<N>() / T;
   const long rows = (long)a.f.nprobe * a.f.nx;
@@ -900,6 +1056,13 @@ hipError_t set_adj_lds_t() {
   if (e == hipSuccess)
     e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_adj_cols<N, false>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, b);
+  const int acc = (int)sizeof(float2) * adj_tpw<N>() * adj_units<N>() * adj_acc_max<N>();
+  if (e == hipSuccess)
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_adj_rows_acc<N, true>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, acc);
+  if (e == hipSuccess)
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_adj_rows_acc<N, false>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, acc);
   return e;
 }
 
