@@ -94,9 +94,29 @@ __device__ __forceinline__ void dft_any(float2* a) {
   }
 }
 
+// W_N^m = exp(-2 pi i m/N) for compile-time m (folded to a constant): m/N turns reduced to
+// the nearest quarter turn and a remainder |a| <= pi/4 whose sine and cosine come from
+// their Taylor series in double precision (degrees 15 and 16, truncation below 1e-16),
+// rounded once.
+template <int N>
+__device__ __forceinline__ float2 twiddle_const(int m) {
+  const int q = (4 * m + N / 2) / N;
+  const double a = (double)(4 * m - q * N) * (3.14159265358979323846 / (2.0 * N)), a2 = a * a;
+  double sa = 1.0, ca = 1.0;
+#pragma unroll
+  for (int k = 7; k >= 1; k--) sa = 1.0 - sa * a2 / (double)((2 * k) * (2 * k + 1));
+#pragma unroll
+  for (int k = 8; k >= 1; k--) ca = 1.0 - ca * a2 / (double)((2 * k - 1) * (2 * k));
+  sa *= a;
+  const int qq = q & 3;  // (cos, sin) of q pi/2 + a
+  const double c = qq == 0 ? ca : (qq == 1 ? -sa : (qq == 2 ? -ca : sa));
+  const double sn = qq == 0 ? sa : (qq == 1 ? ca : (qq == 2 ? -sa : -ca));
+  return make_float2((float)c, (float)-sn);
+}
+
 // Length R1*R2 DFT in registers (natural order in and out) by one Cooley-Tukey step:
 // input n = R2 n1 + n2, output k = k1 + R1 k2; R1-point DFTs over n1, twiddles
-// W_N^(n2 k1) (constants: twiddle_at of compile-time indices), R2-point DFTs over n2.
+// W_N^(n2 k1) (constants: twiddle_const), R2-point DFTs over n2.
 template <int R1, int R2, int DIR>
 __device__ __forceinline__ void dft_2stage(float2* a) {
   constexpr int N = R1 * R2;
@@ -111,7 +131,7 @@ __device__ __forceinline__ void dft_2stage(float2* a) {
     for (int k1 = 0; k1 < R1; k1++) {
       float2 v = u[k1];
       if ((n2 * k1) % N != 0) {
-        const float2 w = twiddle_at<N>((n2 * k1) % N);
+        const float2 w = twiddle_const<N>((n2 * k1) % N);
         v = DIR < 0 ? cmul(v, w) : cmulc(v, w);
       }
       t[n2 * R1 + k1] = v;

@@ -222,72 +222,127 @@ __device__ __forceinline__ void xform_sync() {
   else __syncthreads();
 }
 
-// W_N^m = exp(-2 pi i m/N), 0 <= m < N, computed instead of loaded: m/N turns is
-// reduced exactly to the nearest quarter turn q/4 and a remainder a with |a| <= pi/4
-// (a = (4m - qN) * pi/(2N): an exact integer times one constant, one rounding),
-// whose sine and cosine come from their Taylor series (degrees 9 and 10, truncation
-// below 2e-9); the quarter turn permutes and negates them.
-template <int N>
-__device__ __forceinline__ float2 twiddle_at(int m) {
-  const int q = (4 * m + N / 2) / N;
-  const float a = (float)(4 * m - q * N) * (float)(3.14159265358979323846 / (2.0 * N));
-  const float a2 = a * a;
-  const float sa = a + a * a2 * fmaf(a2, fmaf(a2, fmaf(a2, 1.0f / 362880.0f, -1.0f / 5040.0f), 1.0f / 120.0f),
-                                     -1.0f / 6.0f);
-  const float ca = fmaf(a2, fmaf(a2, fmaf(a2, fmaf(a2, fmaf(a2, -1.0f / 3628800.0f, 1.0f / 40320.0f),
-                                                   -1.0f / 720.0f), 1.0f / 24.0f), -0.5f), 1.0f);
-  // (cos, sin) of q pi/2 + a
-  const int qq = q & 3;
-  const float c = qq == 0 ? ca : (qq == 1 ? -sa : (qq == 2 ? -ca : sa));
-  const float sn = qq == 0 ? sa : (qq == 1 ? ca : (qq == 2 ? -sa : -ca));
-  return make_float2(c, -sn);
+// ---- twiddled butterflies ------------------------------------------------------
+// A radix-R butterfly of inputs a_k with twiddles w^k evaluates A(z) = sum_k a_k z^k at
+// z = w W_R^q, q < R.  Splitting z^(R/2) = +-c at every level makes it log2(R) stages of
+// radix-2 butterflies u = a + c b, v = a - c b, which take six fused multiply-adds each
+// (v = 2a - u) with the twiddle and the rotation in c: 72 instead of 84 instructions for
+// R = 8, 192 instead of 228 for R = 16.  The node of size R' at offset q0 (points
+// q0 + (R/R') k) splits with c = w^(R'/2) W_R^(q0 R'/2); odd halves differ from their even
+// siblings by a quarter turn, so R/2 constants serve all nodes:
+//   R = 2: w;  4: w^2, w;  8: w^4, w^2, w, w W_8;
+//   16: w^8, w^4, w^2, w^2 W_8, w, w W_8, w W_16, w W_16^3.
+
+// u = a + c b -> a, v = a - c b -> b, with c conjugated for DIR > 0 and a quarter turn in
+// the direction of the transform for ROT.  NU, NV: outputs needed.
+template <int DIR, bool ROT, bool NU = true, bool NV = true>
+__device__ __forceinline__ void bf_tw(float2& a, float2& b, float2 c) {
+  const float cy = DIR < 0 ? c.y : -c.y;
+  float px, py, qx, qy;  // c b = (px bx + py by, qx bx + qy by)
+  if constexpr (!ROT) { px = c.x; py = -cy; qx = cy; qy = c.x; }
+  else if constexpr (DIR < 0) { px = cy; py = c.x; qx = -c.x; qy = cy; }
+  else { px = -cy; py = -c.x; qx = c.x; qy = -cy; }
+  const float2 x = a, y = b;
+  if constexpr (NU) {
+    a.x = fmaf(px, y.x, fmaf(py, y.y, x.x));
+    a.y = fmaf(qx, y.x, fmaf(qy, y.y, x.y));
+    if constexpr (NV) {
+      b.x = fmaf(2.0f, x.x, -a.x);
+      b.y = fmaf(2.0f, x.y, -a.y);
+    }
+  } else if constexpr (NV) {
+    b.x = fmaf(-px, y.x, fmaf(-py, y.y, x.x));
+    b.y = fmaf(-qx, y.x, fmaf(-qy, y.y, x.y));
+  }
 }
 
-// Per-thread twiddles of the twiddled passes.  For small three-pass plans they
-// are loaded once into registers (init) and reused by every transform the
-// thread performs; larger plans compute them on every pass (twiddle_at: no
-// table loads and their latency inside the passes, and no registers held).
+template <int R> constexpr int tw_count() { return R / 2; }
+// Exponents of constant i: w^tw_pow W_R^tw_rot.
+template <int R> constexpr int tw_pow(int i) {
+  if (R == 2) return 1;
+  if (R == 4) return i == 0 ? 2 : 1;
+  if (R == 8) return i == 0 ? 4 : (i == 1 ? 2 : 1);
+  return i == 0 ? 8 : (i == 1 ? 4 : (i < 4 ? 2 : 1));
+}
+template <int R> constexpr int tw_rot(int i) {
+  if (R == 8) return i == 3 ? 1 : 0;
+  if (R == 16) return i == 3 ? 2 : (i == 5 ? 2 : (i == 6 ? 1 : (i == 7 ? 3 : 0)));
+  return 0;
+}
+// Constant (and quarter turn) of the node of size S at offset q0 of a radix-R butterfly.
+template <int R> constexpr int tw_index(int S, int q0) {
+  const int rot = q0 * (S / 2) % (R / 4 > 0 ? R / 4 : 1);  // without the quarter turn
+  for (int i = 0; i < R / 2; i++)
+    if (tw_pow<R>(i) == S / 2 && tw_rot<R>(i) == rot) return i;
+  return -1;
+}
+template <int R> constexpr bool tw_quarter(int S, int q0) { return R >= 4 && q0 * (S / 2) >= R / 4; }
+
+// The node of size S at offset q0, its inputs in a[0], a[1], ..; y[q] receives the outputs.
+template <int R, int S, int Q0, int DIR, int NEED>
+__device__ __forceinline__ void node_tw(float2* a, float2* y, const float2* c) {
+  constexpr int I = tw_index<R>(S, Q0);
+  static_assert(I >= 0, "no constant for this node");
+  constexpr bool ROT = tw_quarter<R>(S, Q0);
+  if constexpr (S == 2) {
+    constexpr int q1 = Q0 + R / 2;
+    bf_tw<DIR, ROT, ((NEED >> Q0) & 1) != 0, ((NEED >> q1) & 1) != 0>(a[0], a[1], c[I]);
+    y[Q0] = a[0];
+    y[q1] = a[1];
+  } else {
+#pragma unroll
+    for (int j = 0; j < S / 2; j++) bf_tw<DIR, ROT>(a[j], a[j + S / 2], c[I]);
+    node_tw<R, S / 2, Q0, DIR, NEED>(a, y, c);
+    node_tw<R, S / 2, Q0 + R / S, DIR, NEED>(a + S / 2, y, c);
+  }
+}
+template <int R, int DIR, int NEED = -1>
+__device__ __forceinline__ void dft_tw(float2* a, const float2* c) {
+  float2 y[R];
+  node_tw<R, R, 0, DIR, NEED>(a, y, c);
+#pragma unroll
+  for (int q = 0; q < R; q++) a[q] = y[q];
+}
+
+// Per-thread constants of the twiddled passes, read once from the table W_N^m and kept in
+// registers (8 to 16 complex values) for every transform the thread performs.  Computing
+// the twiddles in the pass instead (sines and cosines by series, 25 instructions each) was
+// half of the 4096-point row sweep's instructions.
 template <int N>
 struct Twiddles {
   using P = Plan<N>;
   static constexpr int T = N / P::E;
-  static constexpr int NS1 = P::R0, NS2 = P::R0 * P::R1;
-  static constexpr int NB1 = P::E / P::R1, NB2 = P::E / P::R2;
-  static constexpr int C1 = NB1 * (P::R1 - 1), C2 = NB2 * (P::R2 - 1);
-  static constexpr bool REG = P::NP == 3 && (C1 + C2) <= 16;
-  float2 w1[REG ? C1 : 1], w2[REG ? C2 : 1];
-  const float2* tab;  // the table W_N^m, m < N
-  // REG: both twiddled passes' factors from the table, held in registers;
-  // otherwise each pass computes its own (twiddle_at) or loads them from tab
-  __device__ __forceinline__ void init(const float2* __restrict__ tw, int t) {
-    tab = tw;
-    if constexpr (REG) {
+  static constexpr int NS1 = P::R0, NS2 = P::R0 * P::R1, NS3 = P::R0 * P::R1 * P::R2;
+  // butterflies of a pass share their constants when T is a multiple of the span
+  static constexpr int B1 = T % NS1 == 0 ? 1 : P::E / P::R1;
+  static constexpr int B2 = P::NP < 3 ? 0 : (T % NS2 == 0 ? 1 : P::E / P::R2);
+  static constexpr int B3 = P::NP < 4 ? 0 : (T % NS3 == 0 ? 1 : P::E / P::R3);
+  static constexpr int C1 = tw_count<P::R1>(), C2 = tw_count<P::R2>(), C3 = tw_count<P::R3>();
+  float2 w1[B1 * C1], w2[B2 > 0 ? B2 * C2 : 1], w3[B3 > 0 ? B3 * C3 : 1];
+  template <int R, int NS, int B>
+  static __device__ __forceinline__ void load(float2* w, const float2* __restrict__ tw, int t) {
 #pragma unroll
-      for (int b = 0; b < NB1; b++) {
-        const int jm = (t + T * b) % NS1;
+    for (int b = 0; b < B; b++) {
+      const int m = (t + T * b) % NS * (N / (NS * R));
 #pragma unroll
-        for (int k = 1; k < P::R1; k++) w1[b * (P::R1 - 1) + k - 1] = tw[k * jm * (N / (NS1 * P::R1))];
-      }
-#pragma unroll
-      for (int b = 0; b < NB2; b++) {
-        const int jm = (t + T * b) % NS2;
-#pragma unroll
-        for (int k = 1; k < P::R2; k++) w2[b * (P::R2 - 1) + k - 1] = tw[k * jm * (N / (NS2 * P::R2))];
-      }
+      for (int i = 0; i < R / 2; i++) w[b * (R / 2) + i] = tw[tw_pow<R>(i) * m + tw_rot<R>(i) * (N / R)];
     }
+  }
+  __device__ __forceinline__ void init(const float2* __restrict__ tw, int t) {
+    load<P::R1, NS1, B1>(w1, tw, t);
+    if constexpr (P::NP >= 3) load<P::R2, NS2, B2>(w2, tw, t);
+    if constexpr (P::NP >= 4) load<P::R3, NS3, B3>(w3, tw, t);
   }
 };
 
-// One Stockham pass.  FIRST: input from registers (natural layout).  LAST:
+// One Stockham pass.  FIRST: input from registers (natural layout), no twiddles.  LAST:
 // output to registers (natural layout).  Otherwise through the LDS slot.
-// wr: this pass's register twiddles, or nullptr: the pass computes them (TWC)
-// or loads them from tab, the table W_N^m = exp(-2 pi i m/N), m < N.
+// w: the pass's constants (Twiddles), B sets of them over the thread's butterflies.
 // ZIN (first pass) / NEED (last pass): masks over the natural-layout register
 // slots m (element t + T*m) that are zero on input / needed on output; used when
 // one butterfly covers all E slots (R == E), ignored otherwise.
-template <int N, int R, int NS, int DIR, bool FIRST, bool LAST, bool SWZ, int ZIN = 0, int NEED = -1, bool TWC = true>
-__device__ __forceinline__ void stockham_pass(float2* v, float2* slot, const float2* wr,
-                                              const float2* __restrict__ tab, int t) {
+template <int N, int R, int NS, int DIR, bool FIRST, bool LAST, bool SWZ, int B, int ZIN = 0, int NEED = -1>
+__device__ __forceinline__ void stockham_pass(float2* v, float2* slot, const float2* w, int t) {
   constexpr int E = Plan<N>::E;
   constexpr int T = N / E;
   constexpr int NB = E / R;
@@ -303,43 +358,14 @@ __device__ __forceinline__ void stockham_pass(float2* v, float2* slot, const flo
 #pragma unroll
       for (int k = 0; k < R; k++) a[b][k] = slot[lidx<N, SWZ>(t + T * b + k * (N / R))];
   }
-  if constexpr (NS > 1) {
-    // computed or table twiddles are formed where they are used: the empty asm
-    // makes the index offset opaque, so they are not hoisted out of the callers'
-    // loops into registers held across the whole kernel (and the table stays in
-    // the global address space: global loads, not flat ones that also hold up
-    // the LDS waits)
-    int z = 0;
-    if (!wr) asm volatile("" : "+s"(z));
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-      const int jm = (t + T * b) % NS;
-      // w^k of w = W_N^{jm N/(NS R)}: computed or loaded for k < 4 and k a
-      // multiple of 4, the others as w^(k & ~3) * w^(k & 3) (6 evaluations or
-      // loads for a radix-16 pass)
-      float2 pw[R];
-      if (!wr) {
-#pragma unroll
-        for (int k = 1; k < R; k++)
-          if ((k & 3) == 0 || k < 4) {
-            const int m = z + k * jm * (N / (NS * R));
-            pw[k] = TWC ? twiddle_at<N>(m) : tab[m];
-          }
-#pragma unroll
-        for (int k = 5; k < R; k++)
-          if (k & 3) pw[k] = cmul(pw[k & ~3], pw[k & 3]);
-      }
-#pragma unroll
-      for (int k = 1; k < R; k++) {
-        const float2 w = wr ? wr[b * (R - 1) + k - 1] : pw[k];
-        a[b][k] = DIR < 0 ? cmul(a[b][k], w) : cmulc(a[b][k], w);
-      }
-    }
-  }
 #pragma unroll
   for (int b = 0; b < NB; b++) {
-    if constexpr (NB == 1) dft<R, DIR, FIRST ? ZIN : 0, LAST ? NEED : -1>(a[b]);
-    else dft<R, DIR>(a[b]);
+    if constexpr (FIRST) {
+      if constexpr (NB == 1) dft<R, DIR, ZIN>(a[b]);
+      else dft<R, DIR>(a[b]);
+    } else {
+      dft_tw<R, DIR, LAST && NB == 1 ? NEED : -1>(a[b], w + (B > 1 ? b * (R / 2) : 0));
+    }
   }
   if constexpr (LAST) {
 #pragma unroll
@@ -375,19 +401,19 @@ constexpr int gap_mask() {
 // Full length-N transform of the thread-distributed vector v (natural layout
 // in and out).  slot: this transform's LDS region of lds_slot<N, SWZ>() float2.
 // ZIN: slots known to be zero on input; NEED: slots needed on output.
-template <int N, int DIR, bool SWZ = kSwz<N>, int ZIN = 0, int NEED = -1, bool TWC = true>
+template <int N, int DIR, bool SWZ = kSwz<N>, int ZIN = 0, int NEED = -1>
 __device__ __forceinline__ void fft_wave(float2* v, float2* slot, const Twiddles<N>& tw, int t) {
   using P = Plan<N>;
+  using W = Twiddles<N>;
   constexpr int S1 = P::R0;
   constexpr int S2 = P::R0 * P::R1;
-  constexpr bool REG = Twiddles<N>::REG;
-  stockham_pass<N, P::R0, 1, DIR, true, false, SWZ, ZIN, -1, TWC>(v, slot, nullptr, tw.tab, t);
-  stockham_pass<N, P::R1, S1, DIR, false, false, SWZ, 0, -1, TWC>(v, slot, REG ? tw.w1 : nullptr, tw.tab, t);
+  stockham_pass<N, P::R0, 1, DIR, true, false, SWZ, 1, ZIN>(v, slot, nullptr, t);
+  stockham_pass<N, P::R1, S1, DIR, false, false, SWZ, W::B1>(v, slot, tw.w1, t);
   if constexpr (P::NP == 3) {
-    stockham_pass<N, P::R2, S2, DIR, false, true, SWZ, 0, NEED, TWC>(v, slot, REG ? tw.w2 : nullptr, tw.tab, t);
+    stockham_pass<N, P::R2, S2, DIR, false, true, SWZ, W::B2, 0, NEED>(v, slot, tw.w2, t);
   } else {
-    stockham_pass<N, P::R2, S2, DIR, false, false, SWZ, 0, -1, TWC>(v, slot, nullptr, tw.tab, t);
-    stockham_pass<N, P::R3, S2 * P::R2, DIR, false, true, SWZ, 0, NEED, TWC>(v, slot, nullptr, tw.tab, t);
+    stockham_pass<N, P::R2, S2, DIR, false, false, SWZ, W::B2>(v, slot, tw.w2, t);
+    stockham_pass<N, P::R3, S2 * P::R2, DIR, false, true, SWZ, W::B3, 0, NEED>(v, slot, tw.w3, t);
   }
 }
 
