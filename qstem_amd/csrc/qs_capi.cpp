@@ -718,6 +718,7 @@ static int bl_sweeps(qs_ctx* c, float2* tr, int nslice, const float* vpot, float
   a.ny = ny;
   a.kc = c->bl.kc;
   a.kcp = c->bl.kcp;
+  a.lb = qs::col_line_of(nx);
   a.band_a = c->bl.band_a;
   a.band_b = c->bl.band_b;
   a.ntiles = c->bl.ntiles;
@@ -1391,6 +1392,7 @@ static void fill_sweep_args(qs_ctx* c, RunPlan& r, const int* d_ipos, const int*
   a.ny = p.ny;
   a.kc = c->kc;
   a.kcp = c->kcp;
+  a.lb = qs::col_line_of(p.nx);
   a.band_a = c->band_a;
   a.band_b = c->band_b;
   a.ntiles = c->ntiles;
@@ -2030,7 +2032,7 @@ static void sweep_args(qs_ctx* c, SweepArgs& a, int nprobe) {
   const qs_params& p = c->p;
   a = SweepArgs{};
   a.nx = p.nx; a.ny = p.ny; a.nprobe = nprobe; a.probe0 = 0;
-  a.kc = c->kc; a.kcp = c->kcp; a.band_a = c->band_a; a.band_b = c->band_b; a.ntiles = c->ntiles;
+  a.kc = c->kc; a.kcp = c->kcp; a.lb = qs::col_line_of(p.nx); a.band_a = c->band_a; a.band_b = c->band_b; a.ntiles = c->ntiles;
   a.potNy = p.potNy;
   a.rw = c->rows_per_wave;
   a.tpb = c->tiles_per_block;
@@ -2445,7 +2447,7 @@ int qs_atom_gradients(qs_ctx* c, const qs_atom* atoms, int natom, const qs_pot_p
 // are ignored).
 namespace {
 // bumped whenever the sweep kernels or their launch parameters change meaning
-const char* const kTuneVersion = "sweeps-4";
+const char* const kTuneVersion = "sweeps-5";
 struct TuneKey {
   std::string device;  // gcnArchName / name / compute units
   int nx, ny, kcp, potNy, nstreams;

@@ -112,10 +112,15 @@ __device__ __forceinline__ void dft8(float2* a) {
   if constexpr ((O & 0x80) != 0) a[7] = csub(e3, o3);
 }
 
+// cos and sin of pi/8, and the next larger float of the cosine: the nearest one loses 2.9e-8
+// of the modulus, the next gains 2.7e-8, and what every transform loses adds up over a run.
+// The transforms below use the next one often enough to balance the losses at pi/8 and pi/4.
+constexpr float kCos16 = 0.92387953251128675613f, kCos16Up = 0x1.d906bep-1f, kSin16 = 0.38268343236508977173f;
+
 template <int DIR, int Z = 0>
 __device__ __forceinline__ void dft16(float2* a) {
   // 16 = 4 x 4: columns of stride 4, twiddles W16^{n1 k2}, rows of length 4
-  const float c1 = 0.92387953251128675613f, s1 = 0.38268343236508977173f;
+  const float c1 = kCos16, cu = kCos16Up, s1 = kSin16;
   const float h = 0.70710678118654752440f;
   float2 b[16];
   auto colz = [](int n1) constexpr {
@@ -133,8 +138,8 @@ __device__ __forceinline__ void dft16(float2* a) {
   col(std::integral_constant<int, 3>{});
   // twiddle b[n1*4+k2] *= W16^{n1*k2}
   const float sg = (float)DIR;
-  const float2 w1 = make_float2(c1, sg * s1), w2 = make_float2(h, sg * h), w3 = make_float2(s1, sg * c1);
-  const float2 w6 = make_float2(-h, sg * h), w9 = make_float2(-c1, -sg * s1);
+  const float2 w1 = make_float2(c1, sg * s1), w2 = make_float2(h, sg * h), w3 = make_float2(s1, sg * cu);
+  const float2 w6 = make_float2(-h, sg * h), w9 = make_float2(-cu, -sg * s1);
   b[1 * 4 + 1] = cmul(b[5], w1);
   b[1 * 4 + 2] = cmul(b[6], w2);
   b[1 * 4 + 3] = cmul(b[7], w3);
@@ -256,7 +261,6 @@ __device__ __forceinline__ void bf_tw(float2& a, float2& b, float2 c) {
   }
 }
 
-template <int R> constexpr int tw_count() { return R / 2; }
 // Exponents of constant i: w^tw_pow W_R^tw_rot.
 template <int R> constexpr int tw_pow(int i) {
   if (R == 2) return 1;
@@ -308,16 +312,25 @@ __device__ __forceinline__ void dft_tw(float2* a, const float2* c) {
 // registers (8 to 16 complex values) for every transform the thread performs.  Computing
 // the twiddles in the pass instead (sines and cosines by series, 25 instructions each) was
 // half of the 4096-point row sweep's instructions.
-template <int N>
+// LEAN: only the powers of w are kept (log2(R) per butterfly); the constants turned by W_8
+// or W_16 are multiplied out where used (16 instructions beside the 192 of a radix-16
+// butterfly), which keeps E = 16 transforms with more state of their own at 128 registers.
+template <int N, class PLAN = Plan<N>, bool LEAN = false>
 struct Twiddles {
-  using P = Plan<N>;
+  using P = PLAN;
   static constexpr int T = N / P::E;
   static constexpr int NS1 = P::R0, NS2 = P::R0 * P::R1, NS3 = P::R0 * P::R1 * P::R2;
   // butterflies of a pass share their constants when T is a multiple of the span
   static constexpr int B1 = T % NS1 == 0 ? 1 : P::E / P::R1;
   static constexpr int B2 = P::NP < 3 ? 0 : (T % NS2 == 0 ? 1 : P::E / P::R2);
   static constexpr int B3 = P::NP < 4 ? 0 : (T % NS3 == 0 ? 1 : P::E / P::R3);
-  static constexpr int C1 = tw_count<P::R1>(), C2 = tw_count<P::R2>(), C3 = tw_count<P::R3>();
+  template <int R> static constexpr int per() {  // constants kept per butterfly
+    if (!LEAN) return R / 2;
+    int n = 0;
+    for (int r = R; r > 1; r >>= 1) n++;
+    return n;
+  }
+  static constexpr int C1 = per<P::R1>(), C2 = per<P::R2>(), C3 = per<P::R3>();
   float2 w1[B1 * C1], w2[B2 > 0 ? B2 * C2 : 1], w3[B3 > 0 ? B3 * C3 : 1];
   template <int R, int NS, int B>
   static __device__ __forceinline__ void load(float2* w, const float2* __restrict__ tw, int t) {
@@ -325,7 +338,28 @@ struct Twiddles {
     for (int b = 0; b < B; b++) {
       const int m = (t + T * b) % NS * (N / (NS * R));
 #pragma unroll
-      for (int i = 0; i < R / 2; i++) w[b * (R / 2) + i] = tw[tw_pow<R>(i) * m + tw_rot<R>(i) * (N / R)];
+      for (int i = 0, n = 0; i < R / 2; i++)
+        if (!LEAN || tw_rot<R>(i) == 0) w[b * per<R>() + n++] = tw[tw_pow<R>(i) * m + tw_rot<R>(i) * (N / R)];
+    }
+  }
+  // the R/2 constants of butterfly b from those kept
+  template <int R>
+  static __device__ __forceinline__ void consts(const float2* w, int b, float2* c) {
+    w += b * per<R>();
+#pragma unroll
+    for (int i = 0, n = 0; i < R / 2; i++)
+      if (!LEAN || tw_rot<R>(i) == 0) c[i] = w[n++];
+    if constexpr (LEAN && R >= 8) {  // opaque: the products are not kept across transforms
+      constexpr int k = R == 8 ? 2 : 4;
+      asm volatile("" : "+v"(c[k].x), "+v"(c[k].y));
+      if constexpr (R == 16) asm volatile("" : "+v"(c[2].x), "+v"(c[2].y));
+    }
+    if constexpr (LEAN && R == 8) c[3] = w8_1<-1>(c[2]);
+    if constexpr (LEAN && R == 16) {
+      c[3] = w8_1<-1>(c[2]);
+      c[5] = w8_1<-1>(c[4]);
+      c[6] = cmul(c[4], make_float2(kCos16Up, -kSin16));
+      c[7] = cmul(c[4], make_float2(kSin16, -kCos16Up));
     }
   }
   __device__ __forceinline__ void init(const float2* __restrict__ tw, int t) {

@@ -17,6 +17,7 @@ struct SweepArgs {
   int nprobe;          // probes in this launch
   int probe0;          // global index of the first probe of this launch
   int kc, kcp;         // band columns stored per row, and padded row length
+  int lb;              // log2 of the columns per 128-byte line of the state (col_line of nx)
   int band_a, band_b;  // band = iy in [0, band_a] U [ny-band_b, ny-1]
   int ntiles;          // column tiles per probe in sweep B
   int potNy;           // row pitch of the transmission slice
@@ -247,7 +248,8 @@ void launch_gen_rows(const GenRowArgs& a, hipStream_t st);
 void launch_gen_cols(const GenColArgs& a, int ntiles, hipStream_t st);
 
 bool supported_size(int n);
-int col_tile(int nx);
+int col_tile(int nx);  // columns per tile of the column sweeps
+int col_line_of(int nx);
 
 void launch_sweep_rows(const SweepArgs& a, int mode, hipStream_t st);
 void launch_sweep_cols(const SweepArgs& a, bool rec, bool diff, hipStream_t st);

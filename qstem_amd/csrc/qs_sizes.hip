@@ -23,7 +23,8 @@ void QS_CAT(adj_row_shape_, QS_N)(int* group, int* units) {
   *units = adj_units<QS_N>();
 }
 void QS_CAT(adj_cols_, QS_N)(const AdjArgs& a, bool last, hipStream_t st) { launch_adj_cols_t<QS_N>(a, last, st); }
-int QS_CAT(col_tile_, QS_N)() { return ColCfg<QS_N>::TC; }
+int QS_CAT(col_tile_, QS_N)() { return col_tc<QS_N>(); }
+int QS_CAT(col_line_, QS_N)() { return col_line<QS_N>(); }
 void QS_CAT(rows_fft_, QS_N)(float2* d, long nrows, int dir, const float2* tw, float scale, hipStream_t st) {
   if (dir < 0) rows_fft_t<QS_N, -1>(d, nrows, tw, scale, st);
   else rows_fft_t<QS_N, +1>(d, nrows, tw, scale, st);
