@@ -1560,9 +1560,18 @@ static int run_mixed(qs_ctx* c, const int* ipos, const int* config, int nprobe, 
   const qs_params& p = c->p;
   const int nx = p.nx, ny = p.ny;
   const size_t n2 = (size_t)nx * ny, slice = (size_t)p.potNx * p.potNy;
-  // probe group: its state at most 160 MB, resident in the Infinity Cache across the two kernels
-  const int B = c->batch > 0 ? std::min(c->batch, nprobe)
-                             : (int)std::max<size_t>(1, std::min<size_t>(nprobe, (size_t(160) << 20) / (8 * n2)));
+  // probe groups of one size, alternating over two streams (as in qs_run_slices): the in-band
+  // columns of the groups in flight stay in the 256 MB Infinity Cache across the two kernels
+  int B = c->batch > 0 ? std::min(c->batch, nprobe) : nprobe;
+  if (c->batch <= 0) {
+    const size_t budget = (size_t)(c->nstreams > 1 ? 96u : 180u) << 20;
+    const int most = (int)std::max<size_t>(1, budget / (sizeof(float2) * (size_t)nx * c->kc));
+    int groups = (nprobe + most - 1) / most;
+    if (c->nstreams > 1) groups = std::max(groups, std::min(2, nprobe));
+    B = (nprobe + groups - 1) / groups;
+  }
+  const int ngroup = (nprobe + B - 1) / B;
+  const int nst = (c->nstreams > 1 && ngroup > 1) ? 2 : 1;
   const bool want_det = det && p.ndet > 0;
   hipStream_t st = c->stream;
   HIPCHK(c, c->state.ensure(sizeof(float2) * n2 * nprobe));
@@ -1573,6 +1582,7 @@ static int run_mixed(qs_ctx* c, const int* ipos, const int* config, int nprobe, 
     HIPCHK(c, hipMemcpyAsync(c->cfgidx.p, config, sizeof(int) * nprobe, hipMemcpyHostToDevice, st));
   }
   HIPCHK(c, c->partial.ensure(sizeof(float) * (size_t)B * c->gntiles * (qs::kMaxDet + 1)));
+  if (nst > 1) HIPCHK(c, c->partial2.ensure(sizeof(float) * (size_t)B * c->gntiles * (qs::kMaxDet + 1)));
   const size_t nd = want_det ? (size_t)nbins * p.ndet * nprobe : 0;
   if (want_det) {
     HIPCHK(c, c->det.ensure(sizeof(float) * nd));
@@ -1618,35 +1628,46 @@ static int run_mixed(qs_ctx* c, const int* ipos, const int* config, int nprobe, 
     ca.det_k2in[d] = c->det_k2in[d];
     ca.det_k2out[d] = c->det_k2out[d];
   }
-  ca.partial = c->partial.as<float>();
   ca.diff_scale = (float)pow((double)n2, 1.5);
   ca.plan = c->gpx;
   ca.tw = c->twx.as<float2>();
-  for (int p0 = 0; p0 < nprobe; p0 += B) {
+  // launches of the group from probe p0 at slice s; the exit waves follow the last slice
+  auto enqueue = [&](int p0, int s, int k) {
+    hipStream_t gs = k ? c->stream2 : st;
     const int nb = std::min(B, nprobe - p0);
     ra.nprobe = ca.nprobe = nb;
     ra.probe0 = ca.probe0 = p0;
-    for (int s = 0; s < nslice; s++) {
-      ra.mode = (s == 0 && start == 0) ? 0 : 1;
-      ra.trans = trans_base(c) + (size_t)(slice0 + s) * slice;
-      if (c->gvy == qs::kGenPlanCompiled) qs::launch_mix_rows(ra, st);
-      else qs::launch_gen_rows(ra, st);
-      const int bin = want_det && bins ? bins[s] : -1;
-      const bool last = s == nslice - 1, tot = last && int_intensity;
-      ca.rec = (bin >= 0 || tot) ? 1 : 0;
-      ca.diff = (last && diff) ? c->diff.as<float>() : nullptr;
-      if (c->gvx == qs::kGenPlanCompiled) qs::launch_mix_cols(ca, c->gntiles, st);
-      else qs::launch_gen_cols(ca, c->gntiles, st);
-      if (ca.rec)
-        qs::launch_reduce_partials(ca.partial, nb, c->gntiles, bin >= 0 ? p.ndet : 0, p.electronScale,
-                                   bin >= 0 ? c->det.as<float>() + (size_t)bin * p.ndet * nprobe : nullptr, nprobe,
-                                   tot ? c->total.as<float>() : nullptr, p0, st);
-    }
-    if (exit_wave) {  // the real-space exit waves: y-IFFT of the state, no transmit
+    ca.partial = (k ? c->partial2 : c->partial).as<float>();
+    ra.mode = (s == 0 && start == 0) ? 0 : 1;
+    ra.trans = trans_base(c) + (size_t)(slice0 + s) * slice;
+    if (c->gvy == qs::kGenPlanCompiled) qs::launch_mix_rows(ra, gs);
+    else qs::launch_gen_rows(ra, gs);
+    const int bin = want_det && bins ? bins[s] : -1;
+    const bool last = s == nslice - 1, tot = last && int_intensity;
+    ca.rec = (bin >= 0 || tot) ? 1 : 0;
+    ca.diff = (last && diff) ? c->diff.as<float>() : nullptr;
+    if (c->gvx == qs::kGenPlanCompiled) qs::launch_mix_cols(ca, c->gntiles, gs);
+    else qs::launch_gen_cols(ca, c->gntiles, gs);
+    if (ca.rec)
+      qs::launch_reduce_partials(ca.partial, nb, c->gntiles, bin >= 0 ? p.ndet : 0, p.electronScale,
+                                 bin >= 0 ? c->det.as<float>() + (size_t)bin * p.ndet * nprobe : nullptr, nprobe,
+                                 tot ? c->total.as<float>() : nullptr, p0, gs);
+    if (last && exit_wave) {  // the real-space exit waves: y-IFFT of the state, no transmit
       ra.mode = 2;
-      if (c->gvy == qs::kGenPlanCompiled) qs::launch_mix_rows(ra, st);
-      else qs::launch_gen_rows(ra, st);
+      if (c->gvy == qs::kGenPlanCompiled) qs::launch_mix_rows(ra, gs);
+      else qs::launch_gen_rows(ra, gs);
     }
+  };
+  if (nst == 2) {  // the second stream starts after the uploads on the first
+    HIPCHK(c, hipEventRecord(c->evfork, st));
+    HIPCHK(c, hipStreamWaitEvent(c->stream2, c->evfork, 0));
+  }
+  for (int g = 0; g < ngroup; g += nst)
+    for (int s = 0; s < nslice; s++)
+      for (int k = 0; k < nst && g + k < ngroup; k++) enqueue((g + k) * B, s, k);
+  if (nst == 2) {  // and the first waits for the second
+    HIPCHK(c, hipEventRecord(c->evjoin, c->stream2));
+    HIPCHK(c, hipStreamWaitEvent(st, c->evjoin, 0));
   }
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipEventRecord(c->ev1, st));

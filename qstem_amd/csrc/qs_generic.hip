@@ -177,7 +177,7 @@ __device__ __forceinline__ void gen_pass(float2* x, int V, int n, int ld, int ns
           a[i][k] = DIR < 0 ? cmul(a[i][k], w) : cmulc(a[i][k], w);
         }
       }
-      dft_any<R, DIR>(a[i]);
+      dft_any<R, DIR, false>(a[i]);
       dsto[i] = (v << 16) | (q * ns * R + jm);  // vector (< 16) and output element (< 2^16)
     }
   }
@@ -444,39 +444,50 @@ void launch_gen_rowxform(const GenRowXformArgs& a, int dir, hipStream_t st) {
 }
 
 // ============================================================================
-// Compiled-plan sweeps (qs_mix.hpp, one translation unit per length): dispatch.
-#define QS_MIX_DECL(n)                                                   \
-  void mix_rows_##n(const GenRowArgs& a, hipStream_t st);                \
-  void mix_cols_##n(const GenColArgs& a, int nblocks, hipStream_t st);   \
-  int mix_cpb_##n();
+// Compiled-plan sweeps (qs_pair.hpp and qs_mix.hpp, one translation unit per length): dispatch.
+#define QS_DECL(k, n)                                                    \
+  void k##_rows_##n(const GenRowArgs& a, hipStream_t st);                \
+  void k##_cols_##n(const GenColArgs& a, int nblocks, hipStream_t st);   \
+  int k##_cpb_##n();
+#define QS_PAIR_DECL(n) QS_DECL(pair, n)
+#define QS_MIX_DECL(n) QS_DECL(mix, n)
+QS_PAIR_SIZES(QS_PAIR_DECL)
 QS_MIX_SIZES(QS_MIX_DECL)
+#undef QS_PAIR_DECL
 #undef QS_MIX_DECL
+#undef QS_DECL
 
-bool mix_compiled(int n) {
-#define QS_MIX_CASE(m) if (n == m) return true;
-  QS_MIX_SIZES(QS_MIX_CASE)
-#undef QS_MIX_CASE
-  return false;
+namespace {
+struct CompiledPlan {
+  int n;
+  void (*rows)(const GenRowArgs&, hipStream_t);
+  void (*cols)(const GenColArgs&, int, hipStream_t);
+  int (*cpb)();
+};
+#define QS_PAIR_ROW(n) {n, pair_rows_##n, pair_cols_##n, pair_cpb_##n},
+#define QS_MIX_ROW(n) {n, mix_rows_##n, mix_cols_##n, mix_cpb_##n},
+const CompiledPlan kCompiled[] = {QS_PAIR_SIZES(QS_PAIR_ROW) QS_MIX_SIZES(QS_MIX_ROW)};
+#undef QS_PAIR_ROW
+#undef QS_MIX_ROW
+// The plan of length n, or null; of two, the two-pass one except at 384 (QS_MIX_SIZES).
+const CompiledPlan* compiled_plan(int n) {
+  const CompiledPlan* found = nullptr;
+  for (const CompiledPlan& c : kCompiled)
+    if (c.n == n && (!found || n == 384)) found = &c;
+  return found;
 }
+}  // namespace
+
+bool mix_compiled(int n) { return compiled_plan(n) != nullptr; }
 
 int mix_cols_per_block(int n) {
-#define QS_MIX_CASE(m) if (n == m) return mix_cpb_##m();
-  QS_MIX_SIZES(QS_MIX_CASE)
-#undef QS_MIX_CASE
-  return 0;
+  const CompiledPlan* c = compiled_plan(n);
+  return c ? c->cpb() : 0;
 }
 
-void launch_mix_rows(const GenRowArgs& a, hipStream_t st) {
-#define QS_MIX_CASE(m) if (a.ny == m) return mix_rows_##m(a, st);
-  QS_MIX_SIZES(QS_MIX_CASE)
-#undef QS_MIX_CASE
-}
+void launch_mix_rows(const GenRowArgs& a, hipStream_t st) { compiled_plan(a.ny)->rows(a, st); }
 
-void launch_mix_cols(const GenColArgs& a, int nblocks, hipStream_t st) {
-#define QS_MIX_CASE(m) if (a.nx == m) return mix_cols_##m(a, nblocks, st);
-  QS_MIX_SIZES(QS_MIX_CASE)
-#undef QS_MIX_CASE
-}
+void launch_mix_cols(const GenColArgs& a, int nblocks, hipStream_t st) { compiled_plan(a.nx)->cols(a, nblocks, st); }
 
 bool gen_plan(int n, GenPlan* pl) { return gen_plan_variant(n, 0, pl); }
 

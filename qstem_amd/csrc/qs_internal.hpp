@@ -216,15 +216,24 @@ bool gen_plan(int n, GenPlan* pl);  // false: n has a prime factor above 7
 // lengths of mix_compiled only; the GenPlan is then variant 0's, unused)
 constexpr int kGenPlanVariants = 4, kGenPlanCompiled = 3;
 bool gen_plan_variant(int n, int variant, GenPlan* pl);
-// Lengths with a compiled radix plan (qs_mix.hpp; one translation unit qs_mix.hip per
-// length, which the build reads from this list): those measured faster than the
-// runtime-planned kernels (720, 800, 1200 and 1620 have plans too and were not).
-#define QS_MIX_SIZES(X) \
-  X(288) X(300) X(320) X(360) X(384) X(400) X(441) X(448) X(500) X(540) X(600) X(640) X(768) X(900) X(1280) \
-  X(1350) X(1536) X(1800)
-bool mix_compiled(int n);         // n has a compiled radix plan (QS_MIX_SIZES)
-int mix_cols_per_block(int n);    // band columns per block of k_mix_cols<n>
-// a.rpb: rows per transform slot (k_mix_rows, ny = a.ny)
+// Lengths whose compiled radix plan has up to four passes (qs_mix.hpp; one translation unit
+// qs_mix.hip per length, which the build reads from this list): above the two-pass plans'
+// 1024, those measured faster than the runtime-planned kernels (1200 and 1620 were not);
+// 384, where 24 8 2 takes 2.84 ms for a scan that 16 24 takes 3.19 ms for; and 400.
+#define QS_MIX_SIZES(X) X(384) X(400) X(1280) X(1350) X(1536) X(1800)
+// Lengths with a two-pass plan (qs_pair.hpp, one translation unit qs_pair.hip per length):
+// every product of two of its radices between 64 and 1024 (where a length has both, the
+// faster one runs: compiled_plan).
+#define QS_PAIR_SIZES(X) \
+  X(64) X(72) X(80) X(81) X(90) X(96) X(100) X(108) X(112) X(120) X(126) X(128) X(135) X(140) X(144) X(150) \
+  X(160) X(162) X(168) X(180) X(189) X(192) X(196) X(200) X(210) X(216) X(224) X(225) X(240) X(243) X(250) \
+  X(252) X(256) X(270) X(280) X(288) X(294) X(300) X(315) X(320) X(324) X(336) X(350) X(360) X(375) X(378) \
+  X(384) X(392) X(400) X(405) X(420) X(432) X(441) X(448) X(450) X(480) X(486) X(500) X(504) X(512) X(525) \
+  X(540) X(560) X(567) X(576) X(588) X(600) X(625) X(630) X(640) X(648) X(672) X(675) X(700) X(720) X(729) \
+  X(750) X(756) X(768) X(784) X(800) X(810) X(840) X(864) X(896) X(900) X(960) X(1024)
+bool mix_compiled(int n);         // n has a compiled radix plan (QS_PAIR_SIZES or QS_MIX_SIZES)
+int mix_cols_per_block(int n);    // band columns per block of n's column kernel
+// a.rpb: rows per transform slot (ny = a.ny)
 void launch_mix_rows(const GenRowArgs& a, hipStream_t st);
 // a.tiles: the in-band ky columns (a.tc of them), nblocks = ceil(a.tc / mix_cols_per_block(nx))
 void launch_mix_cols(const GenColArgs& a, int nblocks, hipStream_t st);
