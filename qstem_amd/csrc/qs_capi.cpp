@@ -137,11 +137,19 @@ std::vector<float2> twiddles(int n) {
       t[m] = make_float2(rintf(c0), rintf(s0));
       continue;
     }
+    // neighbouring floats by their bit patterns (both parts are nonzero here)
+    auto step = [](float v, int k) {
+      unsigned u;
+      memcpy(&u, &v, sizeof u);
+      u += k;
+      memcpy(&v, &u, sizeof v);
+      return v;
+    };
     double best = 1e300;
     for (int i = -1; i <= 1; i++)
       for (int k = -1; k <= 1; k++) {
-        const float x = i ? nextafterf(c0, i * 2.0f) : c0, y = k ? nextafterf(s0, k * 2.0f) : s0;
-        const double along = sqrt((double)x * x + (double)y * y) - 1.0, across = (double)x * s - (double)y * c;
+        const float x = step(c0, i), y = step(s0, k);
+        const double along = 0.5 * ((double)x * x + (double)y * y - 1.0), across = (double)x * s - (double)y * c;
         const double cost = 100.0 * along * along + across * across;
         if (cost < best) {
           best = cost;
