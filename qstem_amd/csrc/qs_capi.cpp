@@ -1338,7 +1338,7 @@ int qs_kernel_times(const qs_ctx* c, double* ms_rows, double* ms_cols, long* n_r
 // slices; qs_run_groups interleaves the groups of several contexts slice by slice.
 struct RunPlan {
   qs_ctx* c = nullptr;
-  int nprobe = 0, start = 0, nslice = 0, nbins = 0, B = 0;
+  int nprobe = 0, start = 0, nslice = 0, nbins = 0, B = 0, nst = 1;
   int slice0 = 0;  // first transmission slice of the call
   const int* bins = nullptr;
   bool want_det = false, has_cfg = false;
@@ -1376,6 +1376,15 @@ static int check_run(qs_ctx* c, const char* who, const int* ipos, const int* con
       if (bin_of_slice[s] >= nbins) return fail(c, QS_ERR_ARG, w + ": bin index >= nbins");
   }
   return QS_OK;
+}
+
+// Streams of a run of nprobe probes whose state takes `bytes`: without a set group size, one up
+// to 8 MB, where the launches of a slice take a few us each and the fork, the join and twice
+// as many launches cost more than the overlap gives (one / two streams, 20 slices: 2 probes of
+// 512^2, 3 MB, 391 / 472 us; 8 of 256^2, 3 MB, 317 / 377; 4 of 512^2, 6 MB, 468 / 527; 8 of
+// 512^2, 12 MB, 601 / 576; 32 of 256^2, 12 MB, 552 / 525; 64 of 256^2, 709 / 631).
+static int run_streams(const qs_ctx* c, size_t bytes) {
+  return c->batch > 0 || bytes > (size_t(8) << 20) ? c->nstreams : 1;
 }
 
 // Probe-group size: the library default keeps the wave state of the groups in
@@ -1446,7 +1455,8 @@ static int plan_run(qs_ctx* c, const char* who, const int* ipos, const int* conf
   r.nslice = nslice;
   r.nbins = nbins;
   r.bins = bin_of_slice;
-  r.B = group_size(c, nprobe, c->nstreams);
+  r.nst = run_streams(c, sizeof(float2) * (size_t)nprobe * nx * c->kcp);
+  r.B = group_size(c, nprobe, r.nst);
   r.want_det = det && p.ndet > 0;
   r.det = det;
   r.diff = diff;
@@ -1464,7 +1474,7 @@ static int plan_run(qs_ctx* c, const char* who, const int* ipos, const int* conf
     HIPCHK(c, hipMemcpyAsync(c->cfgidx.p, config, sizeof(int) * nprobe, hipMemcpyHostToDevice, c->stream));
   }
   HIPCHK(c, c->partial.ensure(sizeof(float) * (size_t)r.B * c->ntiles * (qs::kMaxDet + 1)));
-  if (c->nstreams > 1 && r.nprobe > r.B)
+  if (r.nst > 1 && r.nprobe > r.B)
     HIPCHK(c, c->partial2.ensure(sizeof(float) * (size_t)r.B * c->ntiles * (qs::kMaxDet + 1)));
   if (r.want_det) {
     const size_t nd = (size_t)nbins * p.ndet * nprobe;
@@ -1570,16 +1580,17 @@ static int run_mixed(qs_ctx* c, const int* ipos, const int* config, int nprobe, 
   const size_t n2 = (size_t)nx * ny, slice = (size_t)p.potNx * p.potNy;
   // probe groups of one size, alternating over two streams (as in qs_run_slices): the in-band
   // columns of the groups in flight stay in the 256 MB Infinity Cache across the two kernels
+  const int streams = run_streams(c, sizeof(float2) * (size_t)nprobe * nx * c->kc);
   int B = c->batch > 0 ? std::min(c->batch, nprobe) : nprobe;
   if (c->batch <= 0) {
-    const size_t budget = (size_t)(c->nstreams > 1 ? 96u : 180u) << 20;
+    const size_t budget = (size_t)(streams > 1 ? 96u : 180u) << 20;
     const int most = (int)std::max<size_t>(1, budget / (sizeof(float2) * (size_t)nx * c->kc));
     int groups = (nprobe + most - 1) / most;
-    if (c->nstreams > 1) groups = std::max(groups, std::min(2, nprobe));
+    if (streams > 1) groups = std::max(groups, std::min(2, nprobe));
     B = (nprobe + groups - 1) / groups;
   }
   const int ngroup = (nprobe + B - 1) / B;
-  const int nst = (c->nstreams > 1 && ngroup > 1) ? 2 : 1;
+  const int nst = (streams > 1 && ngroup > 1) ? 2 : 1;
   const bool want_det = det && p.ndet > 0;
   hipStream_t st = c->stream;
   HIPCHK(c, c->state.ensure(sizeof(float2) * n2 * nprobe));
@@ -1817,7 +1828,7 @@ int qs_run_slices(qs_ctx* c, const int* ipos, const int* config, int nprobe, int
   // the groups of one stream follow each other, and the launches of a pair of
   // groups are issued slice by slice so that both streams stay fed
   const int ngroup = (r.nprobe + r.B - 1) / r.B;
-  const int nst = (c->nstreams > 1 && ngroup > 1) ? 2 : 1;
+  const int nst = (r.nst > 1 && ngroup > 1) ? 2 : 1;
   auto fork = [&]() -> hipError_t {  // the second stream starts after the uploads on the first
     const hipError_t e = hipEventRecord(c->evfork, c->stream);
     return e != hipSuccess ? e : hipStreamWaitEvent(c->stream2, c->evfork, 0);
