@@ -87,7 +87,7 @@ def build_lib(force=True, jobs=8):
         src = os.path.join(CSRC, "qs_pair.hip")
         obj = os.path.join(OBJ, "qs_pair_%d.o" % n)
         jobs_list.append((obj, [HIPCC] + HIPFLAGS + ["-DQS_PAIR_N=%d" % n, "-c", src, "-o", obj], [src] + headers))
-    for name in ("qs_setup.hip", "qs_capi.cpp", "qs_potential.hip", "qs_adjoint.hip", "qs_generic.hip"):
+    for name in ("qs_setup.hip", "qs_capi.cpp", "qs_potential.hip", "qs_adjoint.hip", "qs_generic.hip", "qs_slab.hip"):
         src = os.path.join(CSRC, name)
         if not os.path.exists(src):
             continue

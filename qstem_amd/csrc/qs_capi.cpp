@@ -274,6 +274,7 @@ struct qs_ctx {
   float adj_loss = 0.f;
   int state_probes = 0;
   bool state_valid = false;
+  bool tuning = false;  // qs_autotune is timing the sweeps
   // optional per-launch timing of the two sweeps (HIP events on the context stream)
   bool profiling = false;
   std::vector<hipEvent_t> evpool;
@@ -1440,9 +1441,20 @@ static void fill_sweep_args(qs_ctx* c, RunPlan& r, const int* d_ipos, const int*
   a.diff_scale = (float)pow((double)p.nx * p.ny, 1.5);
 }
 
+// Whether a qs_run_slices call is one launch of k_slab: windows that one CU holds (per-launch
+// profiling and the autotuner keep the two sweeps, whose times they want).  20 slices, sweeps /
+// k_slab: of 64^2 one probe 220 / 162 us, 128 probes 310 / 166; of 128 x 64 one 255 / 201; of
+// 128^2, where a CU takes as long for a slice as the sweeps' launches, 16 probes 274 / 296, 24
+// 298 / 297, 128 566 / 307.
+static bool slab_run(const qs_ctx* c, int nprobe) {
+  const qs_params& p = c->p;
+  return !c->generic && !c->profiling && !c->tuning && (nprobe >= 24 || p.nx * p.ny < 128 * 128) &&
+         qs::slab_fits(p.nx, p.ny, c->kc);
+}
+
 static int plan_run(qs_ctx* c, const char* who, const int* ipos, const int* config, int nprobe, int start,
                     const int* bin_of_slice, int nslice, int nbins, float* det, float* diff, float* exit_wave,
-                    float* int_intensity, RunPlan& r, int slice0 = 0) {
+                    float* int_intensity, RunPlan& r, int slice0 = 0, bool slab = false) {
   const qs_params& p = c->p;
   const int rc = check_run(c, who, ipos, config, nprobe, start, bin_of_slice, nslice, nbins, det, slice0);
   if (rc != QS_OK) return rc;
@@ -1466,7 +1478,8 @@ static int plan_run(qs_ctx* c, const char* who, const int* ipos, const int* conf
   r.slice_elems = (size_t)p.potNx * p.potNy;
   const size_t state_elems = (size_t)nprobe * nx * c->kcp;
   HIPCHK(c, c->state.ensure(sizeof(float2) * state_elems));
-  if (start == 0) qs::launch_fill_zero(c->state.as<float2>(), state_elems, c->stream);  // padding columns stay zero
+  // padding columns stay zero (k_slab writes them)
+  if (start == 0 && !slab) qs::launch_fill_zero(c->state.as<float2>(), state_elems, c->stream);
   HIPCHK(c, c->ipos.ensure(sizeof(int) * 2 * nprobe));
   HIPCHK(c, hipMemcpyAsync(c->ipos.p, ipos, sizeof(int) * 2 * nprobe, hipMemcpyHostToDevice, c->stream));
   if (config) {
@@ -1545,6 +1558,31 @@ static hipError_t enqueue_slice(RunPlan& r, int p0, int s, hipStream_t st, float
   }
   if (last && r.exit_wave) qs::launch_sweep_rows(a, 2, st);
   return hipSuccess;
+}
+
+// All slices of a planned run of a small window, one block per probe (k_slab), in pieces of
+// kSlabSlices slices that continue from the state.
+static hipError_t enqueue_slab(RunPlan& r, hipStream_t st) {
+  qs_ctx* c = r.c;
+  qs::SlabArgs A{};
+  A.f = r.a;
+  A.f.nprobe = r.nprobe;
+  A.slice_elems = (long long)r.slice_elems;
+  A.escale = c->p.electronScale;
+  A.det = r.det_d;
+  for (int s0 = 0; s0 < r.nslice; s0 += qs::kSlabSlices) {
+    A.nslice = std::min(qs::kSlabSlices, r.nslice - s0);
+    const bool last = s0 + A.nslice == r.nslice;
+    A.start = s0 > 0 ? 1 : r.start;
+    A.f.trans = trans_base(c) + (size_t)(r.slice0 + s0) * r.slice_elems;
+    A.f.out_wave = last && r.exit_wave ? r.exit_d : nullptr;
+    A.f.diff = last && r.diff ? r.diff_d : nullptr;
+    A.total = last && r.intensity ? r.total_d : nullptr;
+    for (int s = 0; s < A.nslice; s++) A.bin[s] = (short)(r.want_det && r.bins ? std::max(r.bins[s0 + s], -1) : -1);
+    const hipError_t e = qs::launch_slab(A, st);
+    if (e != hipSuccess) return e;
+  }
+  return hipGetLastError();
 }
 
 // Device-to-host copies of the requested outputs on stream st (then synchronised).
@@ -1818,16 +1856,17 @@ int qs_run_slices(qs_ctx* c, const int* ipos, const int* config, int nprobe, int
   if (c->generic)
     return run_generic(c, ipos, config, nprobe, start, first_slice, bin_of_slice, nslice, nbins, det, diff,
                        exit_wave, int_intensity);
+  const bool slab = slab_run(c, nprobe) && nbins <= 32767;  // (k_slab's bin numbers are 16-bit)
   RunPlan r;
   int rc = plan_run(c, "qs_run_stem", ipos, config, nprobe, start, bin_of_slice, nslice, nbins, det, diff, exit_wave,
-                    int_intensity, r, first_slice);
+                    int_intensity, r, first_slice, slab);
   if (rc != QS_OK) return rc;
   LaunchMarks lm{c};
   HIPCHK(c, hipEventRecord(c->ev0, c->stream));
   // probe group g runs on stream g % 2 (one stream for a single group or nstreams 1);
   // the groups of one stream follow each other, and the launches of a pair of
   // groups are issued slice by slice so that both streams stay fed
-  const int ngroup = (r.nprobe + r.B - 1) / r.B;
+  const int ngroup = slab ? 1 : (r.nprobe + r.B - 1) / r.B;
   const int nst = (r.nst > 1 && ngroup > 1) ? 2 : 1;
   auto fork = [&]() -> hipError_t {  // the second stream starts after the uploads on the first
     const hipError_t e = hipEventRecord(c->evfork, c->stream);
@@ -1839,6 +1878,7 @@ int qs_run_slices(qs_ctx* c, const int* ipos, const int* config, int nprobe, int
   };
   // launches of stream `only` (or of both streams, only = -1)
   auto enqueue = [&](int only) -> hipError_t {
+    if (slab) return enqueue_slab(r, c->stream);
     hipError_t e = hipSuccess;
     for (int g = 0; g < ngroup; g += nst)
       for (int s = 0; s < r.nslice; s++)
@@ -1858,7 +1898,7 @@ int qs_run_slices(qs_ctx* c, const int* ipos, const int* config, int nprobe, int
                                   (long long)c->diff.p, (long long)c->exitw.p, (long long)c->total.p,
                                   (long long)c->partial.p, (long long)c->partial2.p, nst, (long long)c->ipos.p,
                                   (long long)c->cfgidx.p, (long long)c->probe.p, c->rows_per_wave,
-                                  c->tiles_per_block};
+                                  c->tiles_per_block, slab};
     for (int s = 0; s < nslice; s++) key.push_back(bin_of_slice ? bin_of_slice[s] : -1);
     if (!c->gexec || key != c->gkey) {
       // one graph per stream, each the linear chain of that stream's launches (measured
@@ -2595,6 +2635,7 @@ int qs_autotune(qs_ctx* c, const int* ipos, int nprobe, int* batch, int* rows_pe
     const bool graph = c->use_graph, prof = c->profiling;
     c->use_graph = false;
     c->profiling = false;
+    c->tuning = true;
     // mixed-radix path: rw = rows per block, tpb = columns per tile, vx/vy = plan variants
     int vx = c->gvx, vy = c->gvy;
     auto measure = [&](int B, int rw, int tpb, float* out) -> int {
@@ -2658,6 +2699,7 @@ int qs_autotune(qs_ctx* c, const int* ipos, int nprobe, int* batch, int* rows_pe
     }
     c->use_graph = graph;
     c->profiling = prof;
+    c->tuning = false;
     if (rc != QS_OK) return rc;
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tune_cache[key] = best;

@@ -50,6 +50,23 @@ struct SweepArgs {
   float gv_sigma = 0.f;         // sweep A mode 4: interaction constant sigma
 };
 
+// A whole run of a small window in one launch (qs_slab.hip), up to kSlabSlices slices of it.
+constexpr int kSlabSlices = 512;
+struct SlabArgs {
+  SweepArgs f;             // geometry, tables, probe, ipos, cfg, state, out_wave and diff (nullable), nprobe;
+                           // trans: the first slice
+  int start;               // 1: continue from the state, 0: from the probe
+  int nslice;
+  long long slice_elems;   // elements between consecutive slices
+  float escale;
+  float* det;              // [nbins][ndet][nprobe]
+  float* total;            // nullable: [nprobe] sum |Psi|^2 after the last slice
+  short bin[kSlabSlices];  // detector bin of each slice, -1: none
+};
+bool slab_fits(int nx, int ny, int kc);  // the window has such a kernel
+hipError_t launch_slab(const SlabArgs& a, hipStream_t st);
+hipError_t set_slab_lds();
+
 // Backward sweeps of the adjoint (reverse of SweepArgs' forward sweeps).
 struct AdjArgs {
   SweepArgs f;              // geometry, tables, trans slice, ipos, probe, twiddles

@@ -226,6 +226,7 @@ hipError_t set_col_lds_limits() {
 #define C(N) if ((r = set_col_lds_##N()) != hipSuccess) e = r
   C(64); C(128); C(256); C(512); C(1024); C(2048); C(4096);
 #undef C
+  if ((r = set_slab_lds()) != hipSuccess) e = r;
   return e;
 }
 
