@@ -300,14 +300,16 @@ int qs_adjoint_saved(qs_ctx *ctx, float *grad_V, float *grad_probe);
 int qs_atom_gradients(qs_ctx *ctx, const qs_atom *atoms, int natom, const qs_pot_params *pp, float *grad_xyz);
 
 /* Probes advanced together through all slices before the next group starts
- * (0 = library default).  batch = 1 is the per-probe launch sequence. */
+ * (0 = library default).  batch = 1 is the per-probe launch sequence.  Windows of
+ * 64 and 128 points per side run whole in one launch whatever the group size (at
+ * 128 x 128 from 24 probes; not under qs_set_profiling). */
 int qs_set_batch(qs_ctx *ctx, int batch);
 int qs_get_batch(const qs_ctx *ctx);
 
 /* Streams of qs_run_stem and qs_run_groups: 2 (default) lets consecutive probe
  * groups (qs_run_groups: contexts, by the setting of the first group's context)
  * run on two HIP streams, so that one group's launches fill the other's ramp-up
- * and drain; 1 keeps every launch on the context stream.  Each call waits for
+ * and drain (with the library's group size, once their state exceeds 8 MB); 1 keeps every launch on the context stream.  Each call waits for
  * both streams before it returns.  Results do not depend on it.  No reference
  * counterpart. */
 int qs_set_streams(qs_ctx *ctx, int nstreams);
