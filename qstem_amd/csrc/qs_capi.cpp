@@ -27,6 +27,7 @@
 
 #include "../../include/qstem.h"
 #include "qs_internal.hpp"
+#include "qs_twiddles.hpp"
 
 using qs::ProbeArgs;
 using qs::SweepArgs;
@@ -121,45 +122,8 @@ double wavelength(double kev) {  // stem3/stemutil.cpp:714-725
   return hc / sqrt(kev * (2.0 * emass + kev));
 }
 
-// W_n^m = exp(-2 pi i m/n) rounded to single precision with its modulus kept: of the nine
-// neighbouring pairs of floats, the one whose squared error along the value, weighted 100
-// to 1 against the error across it, is least.  A modulus error is a gain that every
-// transform applies again (rounding both parts to nearest, a 512-point transform loses
-// 2.4e-8 to 3e-8 of the amplitude, and the sum over the slices of a run was the largest
-// error of its detector sums; so rounded, 1.2e-8), an error across it is noise (a
-// transform's rms error grows by 4%).
-std::vector<float2> twiddles(int n) {
-  std::vector<float2> t(n);
-  for (int m = 0; m < n; m++) {
-    const double a = -2.0 * M_PI * m / n, c = cos(a), s = sin(a);
-    const float c0 = (float)c, s0 = (float)s;
-    t[m] = make_float2(c0, s0);
-    if (4LL * m % n == 0) {  // quarter turns are exact
-      t[m] = make_float2(rintf(c0), rintf(s0));
-      continue;
-    }
-    // neighbouring floats by their bit patterns (both parts are nonzero here)
-    auto step = [](float v, int k) {
-      unsigned u;
-      memcpy(&u, &v, sizeof u);
-      u += k;
-      memcpy(&v, &u, sizeof v);
-      return v;
-    };
-    double best = 1e300;
-    for (int i = -1; i <= 1; i++)
-      for (int k = -1; k <= 1; k++) {
-        const float x = step(c0, i), y = step(s0, k);
-        const double along = 0.5 * ((double)x * x + (double)y * y - 1.0), across = (double)x * s - (double)y * c;
-        const double cost = 100.0 * along * along + across * across;
-        if (cost < best) {
-          best = cost;
-          t[m] = make_float2(x, y);
-        }
-      }
-  }
-  return t;
-}
+std::vector<float2> twiddles(int n) { return qs::twiddles<float2>(n); }
+std::vector<float2> butterfly_twiddles(int n) { return qs::butterfly_twiddles<float2>(n); }
 
 // Row transform of length n for the transmission band limit: either a direct
 // power-of-two Stockham transform or Bluestein through M = 2^k >= 2n-1.
@@ -350,7 +314,7 @@ static int setup_rowxform(qs_ctx* c, RowXform& r, int n) {
   r.gen = false;
   if (is_pow2(n) && n >= 64 && n <= 4096) {
     r.M = 0;
-    HIPCHK(c, upload(r.tw, twiddles(n), c->stream));
+    HIPCHK(c, upload(r.tw, butterfly_twiddles(n), c->stream));
     return QS_OK;
   }
   if (qs::gen_plan(n, &r.plan)) {  // prime factors 2, 3, 5, 7: direct mixed-radix passes
@@ -381,7 +345,7 @@ static int setup_rowxform(qs_ctx* c, RowXform& r, int n) {
                                            " needs a Bluestein length above 4096 (only sizes <= 2048 or powers of two "
                                            "<= 4096 are supported)");
   r.M = M;
-  HIPCHK(c, upload(r.tw, twiddles(M), c->stream));
+  HIPCHK(c, upload(r.tw, r.gen ? twiddles(M) : butterfly_twiddles(M), c->stream));
   for (int dir = -1; dir <= 1; dir += 2) {
     std::vector<float2> ch(n), vh(M);
     std::vector<std::complex<double>> cd(n), v(M, 0.0);
@@ -572,7 +536,9 @@ int qs_create(const qs_params* p, qs_ctx** out) {
     c->det_k2in[d] = s0 * s0;
     c->det_k2out[d] = s1 * s1;
   }
-  if (upload(c->twx, twiddles(nx), c->stream) != hipSuccess || upload(c->twy, twiddles(ny), c->stream) != hipSuccess ||
+  // (the sweeps' butterflies; the mixed-radix passes)
+  if (upload(c->twx, fused ? butterfly_twiddles(nx) : twiddles(nx), c->stream) != hipSuccess ||
+      upload(c->twy, fused ? butterfly_twiddles(ny) : twiddles(ny), c->stream) != hipSuccess ||
       upload(c->px, hpx, c->stream) != hipSuccess || upload(c->py, hpy, c->stream) != hipSuccess ||
       upload(c->dkx2, c->kx2, c->stream) != hipSuccess || upload(c->dky2, c->ky2, c->stream) != hipSuccess) {
     c->err = "device allocation of lookup tables failed";

@@ -230,35 +230,27 @@ __device__ __forceinline__ void xform_sync() {
 // ---- twiddled butterflies ------------------------------------------------------
 // A radix-R butterfly of inputs a_k with twiddles w^k evaluates A(z) = sum_k a_k z^k at
 // z = w W_R^q, q < R.  Splitting z^(R/2) = +-c at every level makes it log2(R) stages of
-// radix-2 butterflies u = a + c b, v = a - c b, which take six fused multiply-adds each
-// (v = 2a - u) with the twiddle and the rotation in c: 72 instead of 84 instructions for
-// R = 8, 192 instead of 228 for R = 16.  The node of size R' at offset q0 (points
-// q0 + (R/R') k) splits with c = w^(R'/2) W_R^(q0 R'/2); odd halves differ from their even
-// siblings by a quarter turn, so R/2 constants serve all nodes:
+// radix-2 butterflies u = a + c b, v = a - c b with the twiddle and the rotation in c.  With
+// c = cos (1 + i tan) each takes six fused multiply-adds: b (1 + i tan) in two, and its
+// product with the cosine added to and subtracted from a in four: 72 instead of 84
+// instructions for R = 8, 192 instead of 228 for R = 16.  (v = 2a - u from u = a + c b also
+// takes six, but carries the rounding of u into v: where |u| is much larger than |v|, as for
+// a wave with a large mean, a 4096-point transform's rms error was 30% larger.)  The node of
+// size R' at offset q0 (points q0 + (R/R') k) splits with c = w^(R'/2) W_R^(q0 R'/2); odd
+// halves differ from their even siblings by a quarter turn, so R/2 constants serve all nodes:
 //   R = 2: w;  4: w^2, w;  8: w^4, w^2, w, w W_8;
 //   16: w^8, w^4, w^2, w^2 W_8, w, w W_8, w W_16, w W_16^3.
 
-// u = a + c b -> a, v = a - c b -> b, with c conjugated for DIR > 0 and a quarter turn in
-// the direction of the transform for ROT.  NU, NV: outputs needed.
+// u = a + c b -> a, v = a - c b -> b, with c = (cos, tan) conjugated for DIR > 0 and a quarter
+// turn in the direction of the transform for ROT.  NU, NV: outputs needed.
 template <int DIR, bool ROT, bool NU = true, bool NV = true>
 __device__ __forceinline__ void bf_tw(float2& a, float2& b, float2 c) {
-  const float cy = DIR < 0 ? c.y : -c.y;
-  float px, py, qx, qy;  // c b = (px bx + py by, qx bx + qy by)
-  if constexpr (!ROT) { px = c.x; py = -cy; qx = cy; qy = c.x; }
-  else if constexpr (DIR < 0) { px = cy; py = c.x; qx = -c.x; qy = cy; }
-  else { px = -cy; py = -c.x; qx = c.x; qy = -cy; }
-  const float2 x = a, y = b;
-  if constexpr (NU) {
-    a.x = fmaf(px, y.x, fmaf(py, y.y, x.x));
-    a.y = fmaf(qx, y.x, fmaf(qy, y.y, x.y));
-    if constexpr (NV) {
-      b.x = fmaf(2.0f, x.x, -a.x);
-      b.y = fmaf(2.0f, x.y, -a.y);
-    }
-  } else if constexpr (NV) {
-    b.x = fmaf(-px, y.x, fmaf(-py, y.y, x.x));
-    b.y = fmaf(-qx, y.x, fmaf(-qy, y.y, x.y));
-  }
+  const float t = DIR < 0 ? c.y : -c.y;
+  float2 y = make_float2(fmaf(-t, b.y, b.x), fmaf(t, b.x, b.y));
+  if constexpr (ROT) y = mul_i<DIR>(y);
+  const float2 x = a;
+  if constexpr (NU) a = make_float2(fmaf(c.x, y.x, x.x), fmaf(c.x, y.y, x.y));
+  if constexpr (NV) b = make_float2(fmaf(-c.x, y.x, x.x), fmaf(-c.x, y.y, x.y));
 }
 
 // Exponents of constant i: w^tw_pow W_R^tw_rot.
@@ -288,14 +280,14 @@ __device__ __forceinline__ void node_tw(float2* a, float2* y, const float2* c) {
   constexpr int I = tw_index<R>(S, Q0);
   static_assert(I >= 0, "no constant for this node");
   constexpr bool ROT = tw_quarter<R>(S, Q0);
+  constexpr int q1 = Q0 + R / 2;
+  constexpr bool NU = S > 2 || ((NEED >> Q0) & 1) != 0, NV = S > 2 || ((NEED >> q1) & 1) != 0;
+#pragma unroll
+  for (int j = 0; j < S / 2; j++) bf_tw<DIR, ROT, NU, NV>(a[j], a[j + S / 2], c[I]);
   if constexpr (S == 2) {
-    constexpr int q1 = Q0 + R / 2;
-    bf_tw<DIR, ROT, ((NEED >> Q0) & 1) != 0, ((NEED >> q1) & 1) != 0>(a[0], a[1], c[I]);
     y[Q0] = a[0];
     y[q1] = a[1];
   } else {
-#pragma unroll
-    for (int j = 0; j < S / 2; j++) bf_tw<DIR, ROT>(a[j], a[j + S / 2], c[I]);
     node_tw<R, S / 2, Q0, DIR, NEED>(a, y, c);
     node_tw<R, S / 2, Q0 + R / S, DIR, NEED>(a + S / 2, y, c);
   }
@@ -308,59 +300,32 @@ __device__ __forceinline__ void dft_tw(float2* a, const float2* c) {
   for (int q = 0; q < R; q++) a[q] = y[q];
 }
 
-// Per-thread constants of the twiddled passes, read once from the table W_N^m and kept in
-// registers (8 to 16 complex values) for every transform the thread performs.  Computing
-// the twiddles in the pass instead (sines and cosines by series, 25 instructions each) was
-// half of the 4096-point row sweep's instructions.
-// LEAN: only the powers of w are kept (log2(R) per butterfly); the constants turned by W_8
-// or W_16 are multiplied out where used (16 instructions beside the 192 of a radix-16
-// butterfly), which keeps E = 16 transforms with more state of their own at 128 registers.
-template <int N, class PLAN = Plan<N>, bool LEAN = false>
+// The R/2 constants of a butterfly whose twiddle is w = W_N^m, from the table of W_N^m as
+// (cos, tan) pairs.
+template <int N, int R>
+__device__ __forceinline__ void tw_load(float2* c, const float2* __restrict__ tw, int m) {
+#pragma unroll
+  for (int i = 0; i < R / 2; i++) c[i] = tw[tw_pow<R>(i) * m + tw_rot<R>(i) * (N / R)];
+}
+
+// Per-thread constants of the twiddled passes, read once from the table and kept in registers
+// (8 to 16 complex values) for every transform the thread performs.  Computing the twiddles in
+// the pass instead (sines and cosines by series, 25 instructions each) was half of the
+// 4096-point row sweep's instructions.
+template <int N>
 struct Twiddles {
-  using P = PLAN;
+  using P = Plan<N>;
   static constexpr int T = N / P::E;
   static constexpr int NS1 = P::R0, NS2 = P::R0 * P::R1, NS3 = P::R0 * P::R1 * P::R2;
   // butterflies of a pass share their constants when T is a multiple of the span
   static constexpr int B1 = T % NS1 == 0 ? 1 : P::E / P::R1;
   static constexpr int B2 = P::NP < 3 ? 0 : (T % NS2 == 0 ? 1 : P::E / P::R2);
   static constexpr int B3 = P::NP < 4 ? 0 : (T % NS3 == 0 ? 1 : P::E / P::R3);
-  template <int R> static constexpr int per() {  // constants kept per butterfly
-    if (!LEAN) return R / 2;
-    int n = 0;
-    for (int r = R; r > 1; r >>= 1) n++;
-    return n;
-  }
-  static constexpr int C1 = per<P::R1>(), C2 = per<P::R2>(), C3 = per<P::R3>();
-  float2 w1[B1 * C1], w2[B2 > 0 ? B2 * C2 : 1], w3[B3 > 0 ? B3 * C3 : 1];
+  float2 w1[B1 * (P::R1 / 2)], w2[B2 > 0 ? B2 * (P::R2 / 2) : 1], w3[B3 > 0 ? B3 * (P::R3 / 2) : 1];
   template <int R, int NS, int B>
   static __device__ __forceinline__ void load(float2* w, const float2* __restrict__ tw, int t) {
 #pragma unroll
-    for (int b = 0; b < B; b++) {
-      const int m = (t + T * b) % NS * (N / (NS * R));
-#pragma unroll
-      for (int i = 0, n = 0; i < R / 2; i++)
-        if (!LEAN || tw_rot<R>(i) == 0) w[b * per<R>() + n++] = tw[tw_pow<R>(i) * m + tw_rot<R>(i) * (N / R)];
-    }
-  }
-  // the R/2 constants of butterfly b from those kept
-  template <int R>
-  static __device__ __forceinline__ void consts(const float2* w, int b, float2* c) {
-    w += b * per<R>();
-#pragma unroll
-    for (int i = 0, n = 0; i < R / 2; i++)
-      if (!LEAN || tw_rot<R>(i) == 0) c[i] = w[n++];
-    if constexpr (LEAN && R >= 8) {  // opaque: the products are not kept across transforms
-      constexpr int k = R == 8 ? 2 : 4;
-      asm volatile("" : "+v"(c[k].x), "+v"(c[k].y));
-      if constexpr (R == 16) asm volatile("" : "+v"(c[2].x), "+v"(c[2].y));
-    }
-    if constexpr (LEAN && R == 8) c[3] = w8_1<-1>(c[2]);
-    if constexpr (LEAN && R == 16) {
-      c[3] = w8_1<-1>(c[2]);
-      c[5] = w8_1<-1>(c[4]);
-      c[6] = cmul(c[4], make_float2(kCos16Up, -kSin16));
-      c[7] = cmul(c[4], make_float2(kSin16, -kCos16Up));
-    }
+    for (int b = 0; b < B; b++) tw_load<N, R>(w + b * (R / 2), tw, (t + T * b) % NS * (N / (NS * R)));
   }
   __device__ __forceinline__ void init(const float2* __restrict__ tw, int t) {
     load<P::R1, NS1, B1>(w1, tw, t);

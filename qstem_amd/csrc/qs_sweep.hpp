@@ -573,10 +573,12 @@ constexpr int col_gap() {
   return m;
 }
 
-template <int N> using ColTwiddles = Twiddles<N, ColPlan<N>, (ColPlan<N>::E > 8)>;
-
-template <int N, int R, int NS, int DIR, bool FIRST, bool LAST, int B, int ZIN = 0, int NEED = -1>
-__device__ __forceinline__ void col_pass(float2* v, float2* tile, const float2* w, int t) {
+// One pass; its butterflies' constants are read from the table tw where they are used.  Held
+// in registers across both transforms of a column they spill at 4096 (128 registers); with the
+// powers of w alone held and the others multiplied out, a pass takes 40 instructions more
+// (per call: one 4096^2 wave 13.5 against 13.3 ms here, its gradient 13.8 against 13.5).
+template <int N, int R, int NS, int DIR, bool FIRST, bool LAST, int ZIN = 0, int NEED = -1>
+__device__ __forceinline__ void col_pass(float2* v, float2* tile, const float2* __restrict__ tw, int t) {
   using C = ColCfg<N>;
   constexpr int E = C::P::E, T = C::T, NB = E / R;
   float2 a[NB][R];
@@ -593,9 +595,11 @@ __device__ __forceinline__ void col_pass(float2* v, float2* tile, const float2* 
       if constexpr (NB == 1) dft<R, DIR, ZIN>(a[b]);
       else dft<R, DIR>(a[b]);
     } else {
-      float2 cs[R / 2];
-      ColTwiddles<N>::template consts<R>(w, B > 1 ? b : 0, cs);
-      dft_tw<R, DIR, LAST && NB == 1 ? NEED : -1>(a[b], cs);
+      float2 c[R / 2];
+      int m = (t + T * b) % NS * (N / (NS * R));
+      asm volatile("" : "+v"(m));  // opaque: loaded here, not hoisted and held across transforms
+      tw_load<N, R>(c, tw, m);
+      dft_tw<R, DIR, LAST && NB == 1 ? NEED : -1>(a[b], c);
     }
   }
   if constexpr (LAST) {
@@ -618,21 +622,20 @@ __device__ __forceinline__ void col_pass(float2* v, float2* tile, const float2* 
 
 // Length-N transform of the block's columns; tile: the block's LDS at this thread's column.
 template <int N, int DIR, int ZIN = 0, int NEED = -1>
-__device__ __forceinline__ void col_fft(float2* v, float2* tile, const ColTwiddles<N>& tw, int t) {
+__device__ __forceinline__ void col_fft(float2* v, float2* tile, const float2* __restrict__ tw, int t) {
   using P = ColPlan<N>;
-  using W = ColTwiddles<N>;
   constexpr int S1 = P::R0, S2 = P::R0 * P::R1;
-  col_pass<N, P::R0, 1, DIR, true, false, 1, ZIN>(v, tile, nullptr, t);
+  col_pass<N, P::R0, 1, DIR, true, false, ZIN>(v, tile, tw, t);
   if constexpr (P::NP == 2) {
-    col_pass<N, P::R1, S1, DIR, false, true, W::B1, 0, NEED>(v, tile, tw.w1, t);
+    col_pass<N, P::R1, S1, DIR, false, true, 0, NEED>(v, tile, tw, t);
   } else {
     static_assert(P::NP == 3, "two or three passes");
-    col_pass<N, P::R1, S1, DIR, false, false, W::B1>(v, tile, tw.w1, t);
-    col_pass<N, P::R2, S2, DIR, false, true, W::B2, 0, NEED>(v, tile, tw.w2, t);
+    col_pass<N, P::R1, S1, DIR, false, false>(v, tile, tw, t);
+    col_pass<N, P::R2, S2, DIR, false, true, 0, NEED>(v, tile, tw, t);
   }
 }
 
-// One thread's part of a column block: its column and row, transform constants and the
+// One thread's part of a column block: its column and row, the transform's table and the
 // state's addressing, and the propagator P = px py (1/(nx ny) folded into px) of its rows,
 // zero outside k2max.  With E = 8, P is kept in registers for every probe of the block;
 // with E = 16 those would cost half the wavefronts, and a bit per row and py are kept.
@@ -647,7 +650,7 @@ struct ColThread {
   unsigned inside = 0;  // bit m: row t + T m lies inside the band
   float2 py;
   const float2* px;
-  ColTwiddles<NX> tw;
+  const float2* __restrict__ tw;
   __device__ __forceinline__ ColThread(const SweepArgs& a, int c0) {
     c = threadIdx.x % C::TC;
     t = threadIdx.x / C::TC;
@@ -657,7 +660,7 @@ struct ColThread {
     static_assert(T % (16 >> LB) == 0, "rows t + T m lie in the same row of their lines");
     voff = row_off(t, LB, a.kcp) + col_off(col, LB);
     rstep = (unsigned)(T * a.kcp) * 8u;
-    tw.init(a.twx, t);
+    tw = a.twx;
     const float ky2 = a.ky2[max(iy, 0)];
     py = a.py[max(iy, 0)];
     px = a.px + t;
@@ -835,8 +838,8 @@ constexpr int col_lds_bytes_t() {
 }
 
 // Probes per block of k_sweep_cols: a.tpb from the caller when > 0, else as many as leave
-// two blocks for every place on the chip, at most 4 (the block's propagator and transform
-// constants are set up once for all of them).
+// two blocks for every place on the chip, at most 4 (the block's propagator is set up once
+// for all of them).
 template <int N>
 int col_probes(const SweepArgs& a) {
   if (a.tpb > 0) return a.tpb;
