@@ -12,21 +12,21 @@ __device__ __forceinline__ float2 rot_i(float2 v) {  // DIR * i * v
   return DIR < 0 ? make_float2(v.y, -v.x) : make_float2(-v.y, v.x);
 }
 
-// UP: the next larger float for one of the two sines, which gains 5e-9 of the modulus per
-// transform where the nearest one loses 6e-9 (what every transform loses adds up over a run).
-template <int DIR, bool UP = false>
-__device__ __forceinline__ void dft3(float2* a) {
-  const float h = 0.86602540378443865f, hu = UP ? 0x1.bb67b0p-1f : h;  // sin(2 pi/3)
+// UP: the next larger float for the sine, which gains 1.6e-8 of the modulus per transform where
+// the nearest one loses 6e-9 (what every transform loses adds up over a run).
+template <int DIR>
+__device__ __forceinline__ void dft3(float2* a, bool up = false) {
+  const float h = up ? 0x1.bb67b0p-1f : 0.86602540378443865f;  // sin(2 pi/3)
   const float2 b = cadd(a[1], a[2]), d = csub(a[1], a[2]);
   const float2 t = make_float2(a[0].x - 0.5f * b.x, a[0].y - 0.5f * b.y);
-  const float2 u = rot_i<DIR>(make_float2(d.x * h, d.y * hu));
+  const float2 u = rot_i<DIR>(cscale(d, h));
   a[0] = cadd(a[0], b);
   a[1] = cadd(t, u);
   a[2] = csub(t, u);
 }
 
-// BAL: the float below the nearest one for half of the products with sin(2 pi/5): the nearest
-// one gains 9e-9 of the modulus per transform, the two together less than 1e-9.
+// BAL: the float below the nearest one for one of the two products with sin(2 pi/5): the
+// nearest one gains 9e-9 of the modulus per transform, the two together less than 1e-9.
 template <int DIR, bool BAL = false>
 __device__ __forceinline__ void dft5(float2* a) {
   const float c1 = 0.30901699437494742f, c2 = -0.80901699437494742f;  // cos(2 pi/5), cos(4 pi/5)
@@ -37,8 +37,8 @@ __device__ __forceinline__ void dft5(float2* a) {
   const float2 a0 = a[0];
   const float2 r1 = make_float2(a0.x + c1 * b1.x + c2 * b2.x, a0.y + c1 * b1.y + c2 * b2.y);
   const float2 r2 = make_float2(a0.x + c2 * b1.x + c1 * b2.x, a0.y + c2 * b1.y + c1 * b2.y);
-  const float2 i1 = rot_i<DIR>(make_float2(s1 * d1.x + s2 * d2.x, u1 * d1.y + s2 * d2.y));
-  const float2 i2 = rot_i<DIR>(make_float2(s2 * d1.x - s1 * d2.x, s2 * d1.y - u1 * d2.y));
+  const float2 i1 = rot_i<DIR>(make_float2(u1 * d1.x + s2 * d2.x, u1 * d1.y + s2 * d2.y));
+  const float2 i2 = rot_i<DIR>(make_float2(s2 * d1.x - s1 * d2.x, s2 * d1.y - s1 * d2.y));
   a[0] = cadd(a0, cadd(b1, b2));
   a[1] = cadd(r1, i1);
   a[4] = csub(r1, i1);
@@ -46,11 +46,11 @@ __device__ __forceinline__ void dft5(float2* a) {
   a[3] = csub(r2, i2);
 }
 
-template <int DIR>
+// BAL: the float above the nearest one for s3 (modulus: -5e-9 -> -2e-9 per transform).
+template <int DIR, bool BAL = false>
 __device__ __forceinline__ void dft7(float2* a) {
   const float c1 = 0.62348980185873353f, c2 = -0.22252093395631440f, c3 = -0.90096886790241913f;
-  // s3: the float above the nearest one (modulus: -5e-9 -> -2e-9 per transform)
-  const float s1 = 0.78183148246802981f, s2 = 0.97492791218182361f, s3 = 0x1.bc4c06p-2f;
+  const float s1 = 0.78183148246802981f, s2 = 0.97492791218182361f, s3 = BAL ? 0x1.bc4c06p-2f : 0.43388373911755812f;
   const float2 b1 = cadd(a[1], a[6]), b2 = cadd(a[2], a[5]), b3 = cadd(a[3], a[4]);
   const float2 d1 = csub(a[1], a[6]), d2 = csub(a[2], a[5]), d3 = csub(a[3], a[4]);
   const float2 a0 = a[0];
@@ -75,13 +75,14 @@ __device__ __forceinline__ void dft7(float2* a) {
 template <int R1, int R2, int DIR, bool BAL = true>
 __device__ __forceinline__ void dft_2stage(float2* a);
 
-// Composite radices as R1 x R2 (the first stage over R1-point DFTs).  BAL: dft3's and dft5's
-// balanced constants, for the compiled plans.
+// Composite radices as R1 x R2 (the first stage over R1-point DFTs).  BAL: balanced constants
+// of the 3-, 5-, 7- and 16-point DFTs, for the compiled plans.  which: index of this DFT
+// among those of its stage (of 3-point ones, every second takes the larger sine).
 template <int R, int DIR, bool BAL = true>
-__device__ __forceinline__ void dft_any(float2* a) {
-  if constexpr (R == 3) dft3<DIR, BAL>(a);
+__device__ __forceinline__ void dft_any(float2* a, int which = 0) {
+  if constexpr (R == 3) dft3<DIR>(a, BAL && (which & 1));
   else if constexpr (R == 5) dft5<DIR, BAL>(a);
-  else if constexpr (R == 7) dft7<DIR>(a);
+  else if constexpr (R == 7) dft7<DIR, BAL>(a);
   else if constexpr (R == 6) dft_2stage<2, 3, DIR, BAL>(a);
   else if constexpr (R == 9) dft_2stage<3, 3, DIR, BAL>(a);
   else if constexpr (R == 10) dft_2stage<2, 5, DIR, BAL>(a);
@@ -97,7 +98,7 @@ __device__ __forceinline__ void dft_any(float2* a) {
   else if constexpr (R == 30) dft_2stage<5, 6, DIR, BAL>(a);
   else {
     static_assert(R == 2 || R == 4 || R == 8 || R == 16, "radix without a DFT");
-    dft<R, DIR>(a);
+    dft<R, DIR, 0, -1, BAL>(a);
   }
 }
 
@@ -169,7 +170,7 @@ __device__ __forceinline__ void dft_2stage(float2* a) {
     float2 u[R2];
 #pragma unroll
     for (int n2 = 0; n2 < R2; n2++) u[n2] = t[n2 * R1 + k1];
-    dft_any<R2, DIR, BAL>(u);  // (a first stage of 3 and the twiddles by 6 and 12 lose)
+    dft_any<R2, DIR, BAL>(u, k1);  // (a first stage of 3 and the twiddles by 6 and 12 lose)
 #pragma unroll
     for (int k2 = 0; k2 < R2; k2++) a[k1 + R1 * k2] = u[k2];
   }

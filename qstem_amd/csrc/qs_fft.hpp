@@ -114,13 +114,14 @@ __device__ __forceinline__ void dft8(float2* a) {
 
 // cos and sin of pi/8, and the next larger float of the cosine: the nearest one loses 2.9e-8
 // of the modulus, the next gains 2.7e-8, and what every transform loses adds up over a run.
-// The transforms below use the next one often enough to balance the losses at pi/8 and pi/4.
+// The transforms below (BAL) use the next one often enough to balance the losses at pi/8 and
+// pi/4.
 constexpr float kCos16 = 0.92387953251128675613f, kCos16Up = 0x1.d906bep-1f, kSin16 = 0.38268343236508977173f;
 
-template <int DIR, int Z = 0>
+template <int DIR, int Z = 0, bool BAL = true>
 __device__ __forceinline__ void dft16(float2* a) {
   // 16 = 4 x 4: columns of stride 4, twiddles W16^{n1 k2}, rows of length 4
-  const float c1 = kCos16, cu = kCos16Up, s1 = kSin16;
+  const float c1 = kCos16, cu = BAL ? kCos16Up : kCos16, s1 = kSin16;
   const float h = 0.70710678118654752440f;
   float2 b[16];
   auto colz = [](int n1) constexpr {
@@ -158,12 +159,12 @@ __device__ __forceinline__ void dft16(float2* a) {
 }
 
 // Z, O: zero inputs and needed outputs (dft8 prunes both, dft16 the inputs).
-template <int R, int DIR, int Z = 0, int O = -1>
+template <int R, int DIR, int Z = 0, int O = -1, bool BAL = true>
 __device__ __forceinline__ void dft(float2* a) {
   if constexpr (R == 2) dft2<DIR>(a[0], a[1]);
   else if constexpr (R == 4) dft4z<DIR, Z & 15>(a[0], a[1], a[2], a[3]);
   else if constexpr (R == 8) dft8<DIR, Z & 0xff, O & 0xff>(a);
-  else if constexpr (R == 16) dft16<DIR, Z & 0xffff>(a);
+  else if constexpr (R == 16) dft16<DIR, Z & 0xffff, BAL>(a);
 }
 
 // ---- radix plans -------------------------------------------------------------

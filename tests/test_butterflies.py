@@ -1,6 +1,6 @@
 """The twiddled butterflies of qstem_amd/csrc/qs_fft.hpp compiled for the CPU: each output is as
 exact as its own size allows, also where the inputs share a much larger mean, and the
-(cos, tan) table of their constants."""
+(cos, tan) table of their constants; the DFTs of qs_dft.hpp for the mixed-radix passes."""
 import os
 import subprocess
 
@@ -14,7 +14,7 @@ CSRC = os.path.join(os.path.dirname(HERE), "qstem_amd", "csrc")
 @pytest.fixture(scope="module")
 def harness(tmp_path_factory):
     exe = str(tmp_path_factory.mktemp("butterfly") / "harness")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-I" + os.path.join(HERE, "hip_host"), "-I" + CSRC,
+    subprocess.run(["g++", "-std=c++17", "-O1", "-ffp-contract=off", "-I" + os.path.join(HERE, "hip_host"), "-I" + CSRC,
                     os.path.join(HERE, "butterfly_harness.cpp"), "-o", exe], check=True)
 
     def call(text):
@@ -62,3 +62,43 @@ def test_table_of_cosines_and_tangents(harness, n):
         near = near * (1 + 1j * (exact.imag / exact.real).astype(np.float32).astype(np.float64))
     ok = np.abs(exact.real) > 1e-9
     assert np.sum((np.abs(w) - 1)[ok] ** 2) <= np.sum((np.abs(near) - 1)[ok] ** 2)
+
+
+RADICES = [3, 5, 6, 7, 8, 9, 10, 12, 14, 15, 16, 18, 20, 21, 24, 25, 28, 30]
+
+
+def _dft(harness, radix, balanced, sign, a):
+    a = a.astype(np.complex64)
+    return harness("".join("dft %d %d %d %s\n" % (radix, balanced, sign, " ".join("%.9g %.9g" % (v.real, v.imag) for v in row))
+                           for row in a)).reshape(a.shape)
+
+
+@pytest.mark.parametrize("radix", RADICES)
+@pytest.mark.parametrize("balanced", [0, 1])
+@pytest.mark.parametrize("sign", [-1, 1])
+def test_dft_is_linear_in_complex_factors(harness, radix, balanced, sign):
+    rng = np.random.default_rng(radix)
+    a = (rng.standard_normal((50, radix)) + 1j * rng.standard_normal((50, radix))).astype(np.complex64)
+    got = _dft(harness, radix, balanced, sign, a)
+    k = np.arange(radix)
+    want = a.astype(np.complex128) @ np.exp(sign * 2j * np.pi * np.outer(k, k) / radix)
+    # at most five binary or three larger stages, each with a rounded constant: 2^-24 times
+    # about twenty roundings of the values' size
+    assert np.linalg.norm(got - want) <= 20 * 2.0 ** -24 * np.linalg.norm(want)
+    # the real and the imaginary part go through the same constants, so that i times the input
+    # (exact) gives i times the output, bit for bit
+    assert np.array_equal(_dft(harness, radix, balanced, sign, 1j * a), 1j * got)
+
+
+def test_constants_rounded_to_nearest_where_not_balanced(harness):
+    # the runtime-planned kernels' 7-point DFT: sin(2 pi 3/7) to nearest, the balanced one a step above
+    a = np.zeros((1, 7))
+    a[0, 1] = 1.0
+    near, up = (_dft(harness, 7, b, -1, a)[0] for b in (0, 1))
+    s3 = np.float32(np.sin(6 * np.pi / 7))
+    assert np.float32(-near[3].imag) == s3 and np.float32(-up[3].imag) == np.nextafter(s3, np.float32(2))
+    # 16 points: cos(pi/8) likewise in the turns by 3 and 9 sixteenths alone
+    b = np.zeros((1, 16))
+    b[0, 1] = 1.0
+    near = _dft(harness, 16, 0, -1, b)[0]
+    assert np.max(np.abs(near - np.exp(-2j * np.pi * np.arange(16) / 16))) <= 2.0 ** -25
