@@ -495,9 +495,6 @@ __global__ __launch_bounds__(TileCfg<NX>::BLK) void k_tile_cols(SweepArgs a) {
           if (kx2 < a.k2max && (kx2 + ky2) < a.k2max) v[m] = cmul(cmul(v[m], py), px_of(m));
           else v[m] = make_float2(0.f, 0.f);
         }
-        if constexpr (REC) {
-          detector_sums<NX, TileCfg<NX>>(a, red, iy, t, [&](int m) { return v[m]; });
-        }
         if constexpr (DIFF) {  // fftshifted |Psi|^2/sqrt(nx*ny) of the unnormalised Psi
           float* dp = a.diff + (size_t)pg * a.nx * a.ny;
           const int sy = (iy + a.ny / 2) % a.ny;
@@ -511,6 +508,9 @@ __global__ __launch_bounds__(TileCfg<NX>::BLK) void k_tile_cols(SweepArgs a) {
 #pragma unroll
         for (int m = 0; m < E; m++) v[m] = make_float2(0.f, 0.f);
       }
+      // outside the branch: up to 256 a wavefront holds several columns, whose lanes the sums
+      // gather (padding columns hold zeros)
+      if constexpr (REC) detector_sums<NX, TileCfg<NX>>(a, red, max(iy, 0), t, [&](int m) { return v[m]; });
       fft_wave<NX, +1, false, GAP, -1>(v, col, tw, t);
       xform_sync<NX>();
 #pragma unroll
