@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "../../include/qstem.h"
+#include "qs_copyout.hpp"
 #include "qs_internal.hpp"
 #include "qs_twiddles.hpp"
 
@@ -142,6 +143,26 @@ struct LutArgsHost {
 
 }  // namespace
 
+// The calls of qs::CopyOut.
+struct HipCopies {
+  using Error = hipError_t;
+  using Stream = hipStream_t;
+  using Event = hipEvent_t;
+  static constexpr hipError_t ok = hipSuccess;
+  static hipError_t set_device(int d) { return hipSetDevice(d); }
+  static hipError_t host_alloc(void** p, size_t n) { return hipHostMalloc(p, n, hipHostMallocDefault); }
+  static void host_free(void* p) { (void)hipHostFree(p); }
+  static hipError_t event_create(hipEvent_t* e) { return hipEventCreateWithFlags(e, hipEventDisableTiming); }
+  static void event_destroy(hipEvent_t e) { (void)hipEventDestroy(e); }
+  static hipError_t event_record(hipEvent_t e, hipStream_t s) { return hipEventRecord(e, s); }
+  static hipError_t event_wait(hipEvent_t e) { return hipEventSynchronize(e); }
+  static hipError_t stream_wait(hipStream_t s) { return hipStreamSynchronize(s); }
+  static hipError_t copy(void* dst, const void* src, size_t n, hipStream_t s) {
+    return hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, s);
+  }
+  static void clear_error() { (void)hipGetLastError(); }
+};
+
 struct qs_ctx {
   qs_params p{};
   int device = 0;  // HIP device current at qs_create
@@ -153,9 +174,7 @@ struct qs_ctx {
   int nstreams = 2;
   hipStream_t stream2 = nullptr;
   hipEvent_t evfork = nullptr, evjoin = nullptr;
-  // copy_out's pinned buffers and the events of their transfers
-  void* pinned = nullptr;
-  hipEvent_t evpin[10] = {};
+  qs::CopyOut<HipCopies> copies;  // copy_out's pinned buffers
   float last_ms = 0.f;
   std::string err;
   int batch = 0;
@@ -660,9 +679,7 @@ void qs_destroy(qs_ctx* c) {
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   if (c->evfork) (void)hipEventDestroy(c->evfork);
   if (c->evjoin) (void)hipEventDestroy(c->evjoin);
-  for (hipEvent_t e : c->evpin)
-    if (e) (void)hipEventDestroy(e);
-  if (c->pinned) (void)hipHostFree(c->pinned);
+  c->copies.release();
   if (c->stream) (void)hipStreamDestroy(c->stream);
   if (c->stream2) (void)hipStreamDestroy(c->stream2);
   delete c;
@@ -1558,69 +1575,14 @@ static hipError_t enqueue_slab(RunPlan& r, hipStream_t st) {
   return hipGetLastError();
 }
 
-// Device-to-host copy of a large output to pageable memory, behind the work on st: a few
-// threads take chunks of 1 MB, bring them through pinned buffers of their own (two each, the
-// next chunk's transfer under way while one is copied out) and return when all are copied.
-// The runtime's own pageable copy moves 128 MB in 11 ms (12 GB/s: one thread copies, and
-// takes the page faults of a fresh array), these about 2.5 ms (a 4096^2 exit wave with its
-// run 22.4 -> 13.7 ms).
-// Outputs below 16 MB, and memory the device reaches by itself, keep hipMemcpyAsync.
+// Device-to-host copy of an output on stream st; through pinned buffers (qs_copyout.hpp) unless
+// the device reaches dst by itself.
 static hipError_t copy_out(qs_ctx* c, void* dst, const void* src, size_t bytes, hipStream_t st) {
-  constexpr size_t kChunk = size_t(1) << 20;
-  constexpr int kWorkers = 5;
   hipPointerAttribute_t at{};
   const bool known = hipPointerGetAttributes(&at, dst) == hipSuccess && at.type != hipMemoryTypeUnregistered;
   (void)hipGetLastError();  // an unknown pointer is the ordinary case
-  if (bytes < 16 * kChunk || known) return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
-  if (!c->pinned) {
-    if (hipHostMalloc(&c->pinned, 2 * kWorkers * kChunk, hipHostMallocDefault) != hipSuccess) {
-      (void)hipGetLastError();
-      c->pinned = nullptr;
-      return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
-    }
-    for (hipEvent_t& e : c->evpin)
-      if (const hipError_t r = e ? hipSuccess : hipEventCreateWithFlags(&e, hipEventDisableTiming); r != hipSuccess)
-        return r;
-  }
-  const size_t n = (bytes + kChunk - 1) / kChunk;
-  std::atomic<size_t> next{0};
-  std::atomic<int> failed{(int)hipSuccess};
-  auto work = [&](int w) {
-    size_t at_chunk[2] = {n, n};  // chunk on its way in each buffer
-    hipError_t e = w > 0 ? hipSetDevice(c->device) : hipSuccess;  // (a new thread's current device)
-    for (int b = 0; e == hipSuccess; b ^= 1) {
-      char* const buf = static_cast<char*>(c->pinned) + (2 * w + b) * kChunk;
-      const size_t i = next.fetch_add(1);
-      if (i < n) {  // (this buffer's last chunk was copied out below)
-        e = hipMemcpyAsync(buf, static_cast<const char*>(src) + i * kChunk, std::min(kChunk, bytes - i * kChunk),
-                           hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipEventRecord(c->evpin[2 * w + b], st);
-        at_chunk[b] = i;
-      }
-      const size_t j = at_chunk[b ^ 1];
-      if (e == hipSuccess && j < n) {
-        e = hipEventSynchronize(c->evpin[2 * w + (b ^ 1)]);
-        if (e == hipSuccess)
-          memcpy(static_cast<char*>(dst) + j * kChunk, buf + (b ? -(ptrdiff_t)kChunk : (ptrdiff_t)kChunk),
-                 std::min(kChunk, bytes - j * kChunk));
-        at_chunk[b ^ 1] = n;
-      }
-      if (i >= n && at_chunk[0] >= n && at_chunk[1] >= n) break;
-    }
-    if (e != hipSuccess) failed = (int)e;
-  };
-  std::thread helpers[kWorkers - 1];
-  for (int w = 1; w < kWorkers; w++) {
-    try {
-      helpers[w - 1] = std::thread(work, w);
-    } catch (...) {  // no more threads: the others and the caller take its chunks
-      break;
-    }
-  }
-  work(0);
-  for (std::thread& t : helpers)
-    if (t.joinable()) t.join();
-  return (hipError_t)failed.load();
+  if (known) return HipCopies::copy(dst, src, bytes, st);
+  return c->copies.copy(c->device, dst, src, bytes, st);
 }
 
 // Device-to-host copies of the requested outputs on stream st (then synchronised).
