@@ -246,9 +246,11 @@ struct qs_ctx {
   bool have_probe = false;
   // adjoint
   std::vector<DevBuf> ckpt;
-  DevBuf gx, target, lossp, gT, gprobe, gV, dsum, adj_ipos;
-  DevBuf adj_order, adj_xrange;  // several probes: the reverse row sweep's work by transmission row
-  int adj_chunk = 0, adj_nchunk = 0;
+  DevBuf gx, target, lossp, gT, gprobe, gV, dsum;
+  // window offsets of the probes, and the reverse row sweep's work of several of them
+  // (AdjRowWork): [ranges][offsets][order]
+  DevBuf adj_work;
+  int adj_groups = 0, adj_chunk = 0, adj_nchunk = 0;
   // band limit of dL/dt on the second stream: a second band-compact buffer, events
   // "row sweep wrote buffer b" and "band limit done with buffer b"
   DevBuf blstate2;
@@ -661,8 +663,7 @@ void qs_destroy(qs_ctx* c) {
                     &c->lx.tw, &c->lx.chirp_f, &c->lx.vhat_f, &c->lx.chirp_b, &c->lx.vhat_b,
                     &c->lz.tw, &c->lz.chirp_f, &c->lz.vhat_f, &c->lz.chirp_b, &c->lz.vhat_b,
                     &c->gx, &c->target, &c->lossp, &c->gT, &c->gprobe, &c->gV, &c->dsum,
-                    &c->blpx, &c->blpy, &c->blstate, &c->blstate2, &c->adj_ipos,
-                    &c->adj_order, &c->adj_xrange,
+                    &c->blpx, &c->blpy, &c->blstate, &c->blstate2, &c->adj_work,
                     &c->wx.tw, &c->wx.chirp_f, &c->wx.vhat_f, &c->wx.chirp_b, &c->wx.vhat_b,
                     &c->wy.tw, &c->wy.chirp_f, &c->wy.vhat_f, &c->wy.chirp_b, &c->wy.vhat_b, &c->gscratch, &c->gtiles};
   for (DevBuf* b : bufs) b->release();
@@ -2131,7 +2132,7 @@ static qs::AdjArgs adj_args(qs_ctx* c, int nprobe) {
   const qs_params& p = c->p;
   SweepArgs a;
   sweep_args(c, a, nprobe);
-  a.ipos = c->adj_ipos.as<int2>();
+  a.ipos = c->adj_work.as<int2>() + c->adj_groups;
   a.state = c->state.as<float2>();
   qs::AdjArgs A{};
   A.f = a;
@@ -2145,8 +2146,8 @@ static qs::AdjArgs adj_args(qs_ctx* c, int nprobe) {
   A.single_writer = nprobe == 1 ? (whole ? 2 : 1) : 0;
   A.potNx = p.potNx;
   if (nprobe > 1) {
-    A.order = c->adj_order.as<int>();
-    A.xrange = c->adj_xrange.as<int2>();
+    A.order = c->adj_work.as<int>() + 2 * (c->adj_groups + nprobe);
+    A.xrange = c->adj_work.as<int2>();
     A.chunk = c->adj_chunk;
     A.nchunk = c->adj_nchunk;
   }
@@ -2231,16 +2232,19 @@ static int adj_forward(qs_ctx* c, const char* who, const int* ipos, int nprobe, 
   HIPCHK(c, c->gx.ensure(st_bytes));
   if ((int)c->ckpt.size() < nseg + K) c->ckpt.resize(nseg + K);
   for (int j = 0; j < nseg + K; j++) HIPCHK(c, c->ckpt[j].ensure(st_bytes));  // [0,nseg): X_{jK-1}; [nseg,nseg+K): segment
-  HIPCHK(c, c->adj_ipos.ensure(sizeof(int) * 2 * nprobe));
-  HIPCHK(c, hipMemcpyAsync(c->adj_ipos.p, ipos, sizeof(int) * 2 * nprobe, hipMemcpyHostToDevice, c->stream));
-  AdjRowWork work;  // until the synchronisation below
-  if (nprobe > 1) {
-    work = adj_row_work(p, ipos, nprobe);
-    HIPCHK(c, upload(c->adj_order, work.order, c->stream));
-    HIPCHK(c, upload(c->adj_xrange, work.xrange, c->stream));
-    c->adj_chunk = work.chunk;
-    c->adj_nchunk = work.nchunk;
-  }
+  AdjRowWork work;
+  if (nprobe > 1) work = adj_row_work(p, ipos, nprobe);
+  c->adj_groups = (int)work.xrange.size();
+  c->adj_chunk = work.chunk;
+  c->adj_nchunk = work.nchunk;
+  // one upload (each costs a call of few probes about 10 us), on the host until the
+  // synchronisation below
+  std::vector<int> packed;
+  packed.reserve(2 * ((size_t)c->adj_groups + nprobe) + work.order.size());
+  for (const int2& r : work.xrange) packed.insert(packed.end(), {r.x, r.y});
+  packed.insert(packed.end(), ipos, ipos + 2 * (size_t)nprobe);
+  packed.insert(packed.end(), work.order.begin(), work.order.end());
+  HIPCHK(c, upload(c->adj_work, packed, c->stream));
   const size_t nt = (size_t)nprobe * p.nx * p.ny;
   HIPCHK(c, c->target.ensure(sizeof(float) * nt));
   HIPCHK(c, hipMemcpyAsync(c->target.p, target, sizeof(float) * nt, hipMemcpyDefault, c->stream));

@@ -334,7 +334,9 @@ template <int NX> struct TileCfg {
   static constexpr int STRIDE = ((lds_slot<NX, false>() + 31) / 32) * 32 + 2;
 };
 template <int NX> constexpr bool col_staged() { return NX <= 2048; }
-template <int NX> constexpr bool adj_col_staged() { return NX >= 512 && NX <= 2048; }
+// the reverse column sweep has the staged kernel, the direct one (k_adj_cols), or both
+template <int NX> constexpr bool adj_col_staged() { return NX <= 2048; }
+template <int NX> constexpr bool adj_col_direct() { return NX <= 256 || NX == 4096; }
 
 // Tile staging between the row-major state (TC contiguous complex per row) and
 // the column-major LDS tile (PAD layout); 16-byte accesses (two columns per
@@ -525,8 +527,8 @@ __global__ __launch_bounds__(TileCfg<NX>::BLK) void k_tile_cols(SweepArgs a) {
 }
 
 // ============================================================================
-// Sweep B at 4096, and the reverse column sweep there and up to 256 (reverse sweeps of 1024
-// probes of 256^2: 178 us staged, 137 here; with the loss, 432 and 315).
+// Sweep B at 4096, and the reverse column sweep there and, of many probes, up to 256 (reverse
+// sweeps of 1024 probes of 256^2: 178 us staged, 137 here; with the loss, 432 and 315).
 //
 // A block transforms TC adjacent columns of one probe, T threads per column with E values
 // each: thread (t, c), c fastest, holds rows t + T m of column c.  Its loads and stores are
@@ -837,12 +839,10 @@ constexpr int col_lds_bytes_t() {
   else return (int)sizeof(float2) * ColCfg<N>::LDS;
 }
 
-// Probes per block of k_sweep_cols: a.tpb from the caller when > 0, else as many as leave
-// two blocks for every place on the chip, at most 4 (the block's propagator is set up once
-// for all of them).
+// Probes per block of the direct column kernels: as many as leave two blocks for every place
+// on the chip, at most 4 (the block's propagator is set up once for all of them).
 template <int N>
 int col_probes(const SweepArgs& a) {
-  if (a.tpb > 0) return a.tpb;
   constexpr long by_lds = 163840 / col_lds_bytes_t<N, false>(), by_threads = 2048 / ColCfg<N>::BLK;
   constexpr long places = 256 * (by_lds < by_threads ? by_lds : by_threads);
   return (int)std::max<long>(1, std::min<long>(4, (long)a.nprobe * col_blocks<N>(a) / (2 * places)));
@@ -864,7 +864,7 @@ void launch_cols_t(const SweepArgs& a0, bool rec, bool diff, hipStream_t st) {
     grid = dim3((unsigned)(a.nprobe * ((a.ntiles + a.tpb - 1) / a.tpb)));
     block = dim3(TileCfg<N>::BLK);
   } else {
-    a.tpb = col_probes<N>(a0);
+    a.tpb = a0.tpb > 0 ? a0.tpb : col_probes<N>(a0);
     grid = dim3((unsigned)((a.nprobe + a.tpb - 1) / a.tpb * col_blocks<N>(a)));
     block = dim3(ColCfg<N>::BLK);
   }
@@ -1314,44 +1314,56 @@ void launch_adj_rows_t(const AdjArgs& a, bool first, hipStream_t st) {
   }
 }
 
-template <int N, bool LAST>
-constexpr auto adj_col_kernel() {
-  if constexpr (adj_col_staged<N>()) return &k_tile_adj_cols<N, LAST>;
-  else return &k_adj_cols<N, LAST>;
+// Up to 256 the direct reverse kernel has a longer serial chain (block barriers in every
+// exchange) and half as many blocks: from three blocks per CU on it is the faster one, with the
+// loss, whose target reads it spreads over whole lines, from two (at 64 always).  Staged /
+// direct, us: 256 points, 40 probes 12.1 / 13.5, 60 13.6 / 15.0, 80 17.9 / 16.9; with the loss
+// 30 14.3 / 15.9, 40 16.8 / 16.6, 60 25.7 / 18.8; 128 points, 40 probes 7.4 / 8.0, 120 12.4 /
+// 13.0, 320 19.4 / 16.0; with the loss 60 12.1 / 13.9, 120 20.7 / 15.6; 64 points, 160 probes
+// 5.6 / 6.1, 640 12.3 / 11.4; with the loss 2 7.9 / 6.8, 640 19.3 / 12.8.
+template <int N>
+bool adj_cols_staged_run(const SweepArgs& a, bool last) {
+  if constexpr (!adj_col_direct<N>()) return true;
+  if constexpr (!adj_col_staged<N>()) return false;
+  return (long)a.nprobe * col_blocks<N>(a) < (last ? (N == 64 ? 0 : 512) : 768);
 }
 
 template <int N>
 void launch_adj_cols_t(const AdjArgs& a0, bool last, hipStream_t st) {
   AdjArgs a = a0;
-  dim3 grid, block;
-  if constexpr (adj_col_staged<N>()) {
-    grid = dim3((unsigned)(a.f.nprobe * a.f.ntiles));
-    block = dim3(TileCfg<N>::BLK);
-  } else {
-    a.f.tpb = col_probes<N>(a0.f);
-    grid = dim3((unsigned)((a.f.nprobe + a.f.tpb - 1) / a.f.tpb * col_blocks<N>(a.f)));
-    block = dim3(ColCfg<N>::BLK);
+  if (adj_cols_staged_run<N>(a.f, last)) {
+    if constexpr (adj_col_staged<N>()) {
+      const dim3 grid((unsigned)(a.f.nprobe * a.f.ntiles)), block(TileCfg<N>::BLK);
+      constexpr int lds = col_lds_bytes_t<N, true>();
+      if (last) hipLaunchKernelGGL((k_tile_adj_cols<N, true>), grid, block, lds, st, a);
+      else hipLaunchKernelGGL((k_tile_adj_cols<N, false>), grid, block, lds, st, a);
+    }
+  } else if constexpr (adj_col_direct<N>()) {
+    a.f.tpb = col_probes<N>(a.f);
+    const dim3 grid((unsigned)((a.f.nprobe + a.f.tpb - 1) / a.f.tpb * col_blocks<N>(a.f))), block(ColCfg<N>::BLK);
+    constexpr int lds = col_lds_bytes_t<N, false>();
+    if (last) hipLaunchKernelGGL((k_adj_cols<N, true>), grid, block, lds, st, a);
+    else hipLaunchKernelGGL((k_adj_cols<N, false>), grid, block, lds, st, a);
   }
-  constexpr int lds = col_lds_bytes_t<N, adj_col_staged<N>()>();
-  if (last) hipLaunchKernelGGL((adj_col_kernel<N, true>()), grid, block, lds, st, a);
-  else hipLaunchKernelGGL((adj_col_kernel<N, false>()), grid, block, lds, st, a);
 }
 
 template <int N>
 hipError_t set_adj_lds_t() {
-  const int b = col_lds_bytes_t<N, adj_col_staged<N>()>();
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(adj_col_kernel<N, true>()),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, b);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(adj_col_kernel<N, false>()),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, b);
+  hipError_t e = hipSuccess;
+  auto allow = [&](const void* kernel, int bytes) {
+    if (e == hipSuccess) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  };
+  if constexpr (adj_col_staged<N>()) {
+    allow(reinterpret_cast<const void*>(&k_tile_adj_cols<N, true>), col_lds_bytes_t<N, true>());
+    allow(reinterpret_cast<const void*>(&k_tile_adj_cols<N, false>), col_lds_bytes_t<N, true>());
+  }
+  if constexpr (adj_col_direct<N>()) {
+    allow(reinterpret_cast<const void*>(&k_adj_cols<N, true>), col_lds_bytes_t<N, false>());
+    allow(reinterpret_cast<const void*>(&k_adj_cols<N, false>), col_lds_bytes_t<N, false>());
+  }
   const int acc = (int)sizeof(float2) * adj_tpw<N>() * adj_units<N>() * adj_acc_max<N>();
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_adj_rows_acc<N, true>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, acc);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_adj_rows_acc<N, false>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, acc);
+  allow(reinterpret_cast<const void*>(&k_adj_rows_acc<N, true>), acc);
+  allow(reinterpret_cast<const void*>(&k_adj_rows_acc<N, false>), acc);
   return e;
 }
 
