@@ -562,8 +562,10 @@ __host__ __device__ __forceinline__ int col_blocks(const SweepArgs& a) {
   return (a.ntiles * col_tc<NX>() + ColCfg<NX>::TC - 1) / ColCfg<NX>::TC;
 }
 
-// Wavefronts per SIMD of the column sweeps: two 512-thread blocks per CU at 4096.
-template <int NX> constexpr int col_waves() { return NX >= 1024 ? 4 : 1; }
+// Wavefronts per SIMD of the column sweeps: two 512-thread blocks per CU at 4096; with the loss
+// up to 256 one wavefront more for 28 bytes of scratch (320 probes, us without / with the cap:
+// 128^2 28 / 23, 256^2 106 / 101).
+template <int NX> constexpr int col_waves() { return ColPlan<NX>::E > 8 ? 4 : 1; }
 
 // Slots m of the column plan inside the 2/3 band's gap for every thread (gap_mask).
 template <int NX>
@@ -575,12 +577,43 @@ constexpr int col_gap() {
   return m;
 }
 
-// One pass; its butterflies' constants are read from the table tw where they are used.  Held
-// in registers across both transforms of a column they spill at 4096 (128 registers); with the
-// powers of w alone held and the others multiplied out, a pass takes 40 instructions more
-// (per call: one 4096^2 wave 13.5 against 13.3 ms here, its gradient 13.8 against 13.5).
+// Constants of the twiddled passes.  Two-pass plans hold those of their one twiddled pass in
+// registers for every transform of the block (per launch of 320 probes of 256^2 48 us, read
+// where they are used 51).  At 4096 they are read from the table where they are used: held
+// across both transforms of a column they spill (128 registers), and with the powers of w
+// alone held and the others multiplied out a pass takes 40 instructions more (one 4096^2 wave
+// 13.5 against 13.3 ms here, its gradient 13.8 against 13.5).
+template <int N>
+struct ColTwiddles {
+  using P = ColPlan<N>;
+  static constexpr bool HELD = P::NP == 2;
+  static constexpr int T = N / P::E;
+  const float2* __restrict__ tab;
+  float2 w[HELD ? P::E / 2 : 1];
+  template <int R, int NS>
+  static __device__ __forceinline__ int index(int t, int b) { return (t + T * b) % NS * (N / (NS * R)); }
+  __device__ __forceinline__ void init(const float2* __restrict__ tw, int t) {
+    tab = tw;
+    if constexpr (HELD) {
+#pragma unroll
+      for (int b = 0; b < P::E / P::R1; b++) tw_load<N, P::R1>(w + b * (P::R1 / 2), tw, index<P::R1, P::R0>(t, b));
+    }
+  }
+  template <int R, int NS>
+  __device__ __forceinline__ void get(float2* c, int t, int b) const {
+    if constexpr (HELD) {
+#pragma unroll
+      for (int i = 0; i < R / 2; i++) c[i] = w[b * (R / 2) + i];
+    } else {
+      int m = index<R, NS>(t, b);
+      asm volatile("" : "+v"(m));  // opaque: loaded here, not hoisted and held across transforms
+      tw_load<N, R>(c, tab, m);
+    }
+  }
+};
+
 template <int N, int R, int NS, int DIR, bool FIRST, bool LAST, int ZIN = 0, int NEED = -1>
-__device__ __forceinline__ void col_pass(float2* v, float2* tile, const float2* __restrict__ tw, int t) {
+__device__ __forceinline__ void col_pass(float2* v, float2* tile, const ColTwiddles<N>& tw, int t) {
   using C = ColCfg<N>;
   constexpr int E = C::P::E, T = C::T, NB = E / R;
   float2 a[NB][R];
@@ -598,9 +631,7 @@ __device__ __forceinline__ void col_pass(float2* v, float2* tile, const float2* 
       else dft<R, DIR>(a[b]);
     } else {
       float2 c[R / 2];
-      int m = (t + T * b) % NS * (N / (NS * R));
-      asm volatile("" : "+v"(m));  // opaque: loaded here, not hoisted and held across transforms
-      tw_load<N, R>(c, tw, m);
+      tw.template get<R, NS>(c, t, b);
       dft_tw<R, DIR, LAST && NB == 1 ? NEED : -1>(a[b], c);
     }
   }
@@ -624,7 +655,7 @@ __device__ __forceinline__ void col_pass(float2* v, float2* tile, const float2* 
 
 // Length-N transform of the block's columns; tile: the block's LDS at this thread's column.
 template <int N, int DIR, int ZIN = 0, int NEED = -1>
-__device__ __forceinline__ void col_fft(float2* v, float2* tile, const float2* __restrict__ tw, int t) {
+__device__ __forceinline__ void col_fft(float2* v, float2* tile, const ColTwiddles<N>& tw, int t) {
   using P = ColPlan<N>;
   constexpr int S1 = P::R0, S2 = P::R0 * P::R1;
   col_pass<N, P::R0, 1, DIR, true, false, ZIN>(v, tile, tw, t);
@@ -637,7 +668,7 @@ __device__ __forceinline__ void col_fft(float2* v, float2* tile, const float2* _
   }
 }
 
-// One thread's part of a column block: its column and row, the transform's table and the
+// One thread's part of a column block: its column and row, transform constants and the
 // state's addressing, and the propagator P = px py (1/(nx ny) folded into px) of its rows,
 // zero outside k2max.  With E = 8, P is kept in registers for every probe of the block;
 // with E = 16 those would cost half the wavefronts, and a bit per row and py are kept.
@@ -652,7 +683,7 @@ struct ColThread {
   unsigned inside = 0;  // bit m: row t + T m lies inside the band
   float2 py;
   const float2* px;
-  const float2* __restrict__ tw;
+  ColTwiddles<NX> tw;
   __device__ __forceinline__ ColThread(const SweepArgs& a, int c0) {
     c = threadIdx.x % C::TC;
     t = threadIdx.x / C::TC;
@@ -662,7 +693,7 @@ struct ColThread {
     static_assert(T % (16 >> LB) == 0, "rows t + T m lie in the same row of their lines");
     voff = row_off(t, LB, a.kcp) + col_off(col, LB);
     rstep = (unsigned)(T * a.kcp) * 8u;
-    tw = a.twx;
+    tw.init(a.twx, t);
     const float ky2 = a.ky2[max(iy, 0)];
     py = a.py[max(iy, 0)];
     px = a.px + t;
@@ -840,7 +871,7 @@ constexpr int col_lds_bytes_t() {
 }
 
 // Probes per block of the direct column kernels: as many as leave two blocks for every place
-// on the chip, at most 4 (the block's propagator is set up once for all of them).
+// on the chip, at most 4 (the block's propagator and constants are set up once for all of them).
 template <int N>
 int col_probes(const SweepArgs& a) {
   constexpr long by_lds = 163840 / col_lds_bytes_t<N, false>(), by_threads = 2048 / ColCfg<N>::BLK;
