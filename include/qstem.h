@@ -300,9 +300,11 @@ int qs_adjoint_saved(qs_ctx *ctx, float *grad_V, float *grad_probe);
 int qs_atom_gradients(qs_ctx *ctx, const qs_atom *atoms, int natom, const qs_pot_params *pp, float *grad_xyz);
 
 /* Probes advanced together through all slices before the next group starts
- * (0 = library default).  batch = 1 is the per-probe launch sequence.  Windows of
- * 64 and 128 points per side run whole in one launch whatever the group size (at
- * 128 x 128 from 24 probes; not under qs_set_profiling). */
+ * (0 = library default).  batch = 1 is the per-probe launch sequence.  With the
+ * default, qs_run_stem and qs_run_slices take windows of 64 and 128 points per side
+ * through all slices in one launch (at 128 x 128 from 24 probes; not under
+ * qs_set_profiling); a probe's results on the two sides of that line, and with a set
+ * group size, agree to FP32 rounding. */
 int qs_set_batch(qs_ctx *ctx, int batch);
 int qs_get_batch(const qs_ctx *ctx);
 
@@ -329,8 +331,8 @@ int qs_set_graph(qs_ctx *ctx, int on);
  * (not powers of two, prime factors 2, 3, 5, 7) the two values are the rows per block
  * of the row kernel and the columns per tile of the column kernel (powers of two up
  * to 16 that fit the block's LDS; QS_ERR_ARG otherwise); where a length has a compiled
- * plan (288, 300, 320, 360, 384, 400, 441, 448, 500, 540, 600, 640, 768, 900, 1280, 1350,
- * 1536, 1800:
+ * plan (between 64 and 1024 the products of two of the radices 8, 9, 10, 12, 14, 15, 16,
+ * 18, 20, 21, 24, 25, 27, 28, 30 and 32; 1280, 1350, 1536, 1800:
  * wavefront-resident kernels, the default unless QSTEM_COMPILED_PLANS=0 is set when
  * the context is created) the first is the rows per transform slot of the row kernel
  * and the second is unused.  No reference counterpart. */
@@ -341,7 +343,8 @@ int qs_get_tuning(const qs_ctx *ctx, int *rows_per_wave, int *tiles_per_block, i
  * probe (first 8 slices, up to 512 of the given window offsets) over probe group
  * sizes, row-sweep steps per wavefront and column tiles per block, applies the
  * fastest (as qs_set_batch + qs_set_tuning) and reports it (outputs nullable;
- * rate in probe-slices/s).  On the mixed-radix path it tunes the group size, rows
+ * rate in probe-slices/s).  Windows of 64 and 128 points per side keep the library's
+ * group size (0).  On the mixed-radix path it tunes the group size, rows
  * per block, columns per tile and the radix plan of each axis (few large radices,
  * radix 8, radices up to 8, or the compiled plan where the length has one: results
  * then differ by FP32 rounding only).  Results are cached per device model and wave geometry

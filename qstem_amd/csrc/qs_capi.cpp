@@ -263,7 +263,6 @@ struct qs_ctx {
   float adj_loss = 0.f;
   int state_probes = 0;
   bool state_valid = false;
-  bool tuning = false;  // qs_autotune is timing the sweeps
   // optional per-launch timing of the two sweeps (HIP events on the context stream)
   bool profiling = false;
   std::vector<hipEvent_t> evpool;
@@ -1432,14 +1431,14 @@ static void fill_sweep_args(qs_ctx* c, RunPlan& r, const int* d_ipos, const int*
   a.diff_scale = (float)pow((double)p.nx * p.ny, 1.5);
 }
 
-// Whether a qs_run_slices call is one launch of k_slab: windows that one CU holds (per-launch
-// profiling and the autotuner keep the two sweeps, whose times they want).  20 slices, sweeps /
-// k_slab: of 64^2 one probe 220 / 162 us, 128 probes 310 / 166; of 128 x 64 one 255 / 201; of
-// 128^2, where a CU takes as long for a slice as the sweeps' launches, 16 probes 274 / 296, 24
-// 298 / 297, 128 566 / 307.
+// Whether a qs_run_slices call is one launch of k_slab: windows that one CU holds, with the
+// library's group size (a set one, and per-launch profiling, keep the two sweeps).  20 slices,
+// sweeps / k_slab: of 64^2 one probe 220 / 162 us, 128 probes 310 / 166; of
+// 128 x 64 one 255 / 201; of 128^2, where a CU takes as long for a slice as the sweeps'
+// launches, 16 probes 274 / 296, 24 298 / 297, 128 566 / 307.
 static bool slab_run(const qs_ctx* c, int nprobe) {
   const qs_params& p = c->p;
-  return !c->generic && !c->profiling && !c->tuning && (nprobe >= 24 || p.nx * p.ny < 128 * 128) &&
+  return !c->generic && !c->profiling && c->batch == 0 && (nprobe >= 24 || p.nx * p.ny < 128 * 128) &&
          qs::slab_fits(p.nx, p.ny, c->kc);
 }
 
@@ -2530,7 +2529,7 @@ int qs_atom_gradients(qs_ctx* c, const qs_atom* atoms, int natom, const qs_pot_p
 // are ignored).
 namespace {
 // bumped whenever the sweep kernels or their launch parameters change meaning
-const char* const kTuneVersion = "sweeps-5";
+const char* const kTuneVersion = "sweeps-6";
 struct TuneKey {
   std::string device;  // gcnArchName / name / compute units
   int nx, ny, kcp, potNy, nstreams;
@@ -2540,7 +2539,7 @@ struct TuneKey {
   }
 };
 struct TuneVal {
-  int batch, rw, tpb;
+  int batch, rw, tpb;  // 0: the library's
   float rate;
   int vx, vy;  // mixed-radix plan variants (0 for the power-of-two sweeps)
 };
@@ -2569,7 +2568,7 @@ void tune_load_locked(const std::string& path) {
                ver, dev, &k.nx, &k.ny, &k.kcp, &k.potNy, &k.nstreams, &v.batch, &v.rw, &v.tpb, &v.vx, &v.vy,
                &v.rate) != 13)
       continue;
-    if (strcmp(ver, kTuneVersion) != 0 || v.batch < 1) continue;
+    if (strcmp(ver, kTuneVersion) != 0 || v.batch < 0) continue;
     k.device = dev;
     g_tune_cache.emplace(k, v);  // this process's own measurements win
   }
@@ -2638,7 +2637,6 @@ int qs_autotune(qs_ctx* c, const int* ipos, int nprobe, int* batch, int* rows_pe
     const bool graph = c->use_graph, prof = c->profiling;
     c->use_graph = false;
     c->profiling = false;
-    c->tuning = true;
     // mixed-radix path: rw = rows per block, tpb = columns per tile, vx/vy = plan variants
     int vx = c->gvx, vy = c->gvy;
     auto measure = [&](int B, int rw, int tpb, float* out) -> int {
@@ -2669,10 +2667,16 @@ int qs_autotune(qs_ctx* c, const int* ipos, int nprobe, int* batch, int* rows_pe
     };
     int rc = QS_OK;
     const int Bs[] = {16, 32, 64, 96, 128, 192, 256, 384, 512};
-    for (int B : Bs)
-      if (rc == QS_OK && (B <= n || B == Bs[0])) rc = consider(std::min(B, n), 0, 0);
+    if (!c->generic && qs::slab_fits(c->p.nx, c->p.ny, c->kc)) {
+      rc = consider(0, 0, 0);  // the library's group size, which k_slab runs with
+    } else {
+      for (int B : Bs)
+        if (rc == QS_OK && (B <= n || B == Bs[0])) rc = consider(std::min(B, n), 0, 0);
+    }
     const int B0 = best.batch;
-    if (c->mixed) {
+    if (c->batch == 0 && slab_run(c, n)) {
+      // (one launch: the sweeps' shapes do not enter)
+    } else if (c->mixed) {
       for (int rw : {1, 2, 4, 8, 16})
         if (rc == QS_OK && rw <= qs::gen_max_vectors(c->p.ny)) rc = consider(B0, rw, best.tpb);
       for (int tc : {2, 4, 8, 16})  // (the compiled column kernel has no tiles)
@@ -2702,7 +2706,6 @@ int qs_autotune(qs_ctx* c, const int* ipos, int nprobe, int* batch, int* rows_pe
     }
     c->use_graph = graph;
     c->profiling = prof;
-    c->tuning = false;
     if (rc != QS_OK) return rc;
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tune_cache[key] = best;
