@@ -33,13 +33,13 @@ def _listed(name):
 
 
 def mix_sizes():
-    """Lengths with a compiled mixed-radix plan: the QS_MIX_SIZES list of qs_internal.hpp."""
-    return _listed("QS_MIX_SIZES")
+    """Lengths that run a compiled plan of up to four passes: QS_MIX_RUN of qs_internal.hpp."""
+    return _listed("QS_MIX_RUN")
 
 
 def pair_sizes():
-    """Lengths with a compiled two-pass plan: the QS_PAIR_SIZES list of qs_internal.hpp."""
-    return _listed("QS_PAIR_SIZES")
+    """Lengths that run a compiled two-pass plan: the others of QS_PAIR_SIZES of qs_internal.hpp."""
+    return tuple(n for n in _listed("QS_PAIR_SIZES") if n not in mix_sizes())
 
 
 ARCH = os.environ.get("QS_OFFLOAD_ARCH", "gfx950")

@@ -445,17 +445,12 @@ void launch_gen_rowxform(const GenRowXformArgs& a, int dir, hipStream_t st) {
 
 // ============================================================================
 // Compiled-plan sweeps (qs_pair.hpp and qs_mix.hpp, one translation unit per length): dispatch.
-#define QS_DECL(k, n)                                                    \
-  void k##_rows_##n(const GenRowArgs& a, hipStream_t st);                \
-  void k##_cols_##n(const GenColArgs& a, int nblocks, hipStream_t st);   \
-  int k##_cpb_##n();
-#define QS_PAIR_DECL(n) QS_DECL(pair, n)
-#define QS_MIX_DECL(n) QS_DECL(mix, n)
-QS_PAIR_SIZES(QS_PAIR_DECL)
-QS_MIX_SIZES(QS_MIX_DECL)
-#undef QS_PAIR_DECL
-#undef QS_MIX_DECL
-#undef QS_DECL
+template <int N> void launch_pair_rows_t(const GenRowArgs& a, hipStream_t st);
+template <int N> void launch_pair_cols_t(const GenColArgs& a, int nblocks, hipStream_t st);
+template <int N> int pair_cpb();
+template <int N> void launch_mix_rows_t(const GenRowArgs& a, hipStream_t st);
+template <int N> void launch_mix_cols_t(const GenColArgs& a, int nblocks, hipStream_t st);
+template <int N> int mix_cols_block();
 
 namespace {
 struct CompiledPlan {
@@ -464,17 +459,19 @@ struct CompiledPlan {
   void (*cols)(const GenColArgs&, int, hipStream_t);
   int (*cpb)();
 };
-#define QS_PAIR_ROW(n) {n, pair_rows_##n, pair_cols_##n, pair_cpb_##n},
-#define QS_MIX_ROW(n) {n, mix_rows_##n, mix_cols_##n, mix_cpb_##n},
-const CompiledPlan kCompiled[] = {QS_PAIR_SIZES(QS_PAIR_ROW) QS_MIX_SIZES(QS_MIX_ROW)};
-#undef QS_PAIR_ROW
-#undef QS_MIX_ROW
-// The plan of length n, or null; of two, the two-pass one except at 384 (QS_MIX_SIZES).
+template <int N>
+constexpr CompiledPlan plan_row() {
+  if constexpr (mix_runs(N)) return {N, &launch_mix_rows_t<N>, &launch_mix_cols_t<N>, &mix_cols_block<N>};
+  else return {N, &launch_pair_rows_t<N>, &launch_pair_cols_t<N>, &pair_cpb<N>};
+}
+#define QS_PLAN_ROW(n) plan_row<n>(),
+const CompiledPlan kCompiled[] = {QS_MIX_RUN(QS_PLAN_ROW) QS_PAIR_SIZES(QS_PLAN_ROW)};
+#undef QS_PLAN_ROW
+// The plan of length n, or null.
 const CompiledPlan* compiled_plan(int n) {
-  const CompiledPlan* found = nullptr;
   for (const CompiledPlan& c : kCompiled)
-    if (c.n == n && (!found || n == 384)) found = &c;
-  return found;
+    if (c.n == n) return &c;
+  return nullptr;
 }
 }  // namespace
 

@@ -234,13 +234,19 @@ bool gen_plan(int n, GenPlan* pl);  // false: n has a prime factor above 7
 constexpr int kGenPlanVariants = 4, kGenPlanCompiled = 3;
 bool gen_plan_variant(int n, int variant, GenPlan* pl);
 // Lengths whose compiled radix plan has up to four passes (qs_mix.hpp; one translation unit
-// qs_mix.hip per length, which the build reads from this list): above the two-pass plans'
-// 1024, those measured faster than the runtime-planned kernels (1200 and 1620 were not);
-// 384, where 24 8 2 takes 2.84 ms for a scan that 16 24 takes 3.19 ms for; and 400.
+// qs_mix.hip per length): above the two-pass plans' 1024, those measured faster than the
+// runtime-planned kernels (1200 and 1620 were not); 384; and 400.  QS_MIX_RUN: those that run,
+// which the build reads from this list: at 384 a scan takes 2.84 ms with 24 8 2 and 3.19 ms
+// with 16 24; at 400 the two-pass plan is the faster one (columns 71 against 76 us).
 #define QS_MIX_SIZES(X) X(384) X(400) X(1280) X(1350) X(1536) X(1800)
+#define QS_MIX_RUN(X) X(384) X(1280) X(1350) X(1536) X(1800)
+constexpr bool mix_runs(int n) {
+#define QS_IS(m) n == m ||
+  return QS_MIX_RUN(QS_IS) false;
+#undef QS_IS
+}
 // Lengths with a two-pass plan (qs_pair.hpp, one translation unit qs_pair.hip per length):
-// every product of two of its radices between 64 and 1024 (where a length has both, the
-// faster one runs: compiled_plan).
+// every product of two of its radices between 64 and 1024, which runs unless mix_runs(n).
 #define QS_PAIR_SIZES(X) \
   X(64) X(72) X(80) X(81) X(90) X(96) X(100) X(108) X(112) X(120) X(126) X(128) X(135) X(140) X(144) X(150) \
   X(160) X(162) X(168) X(180) X(189) X(192) X(196) X(200) X(210) X(216) X(224) X(225) X(240) X(243) X(250) \
