@@ -625,7 +625,7 @@ def main():
         "tuning": tuning,
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": "slice step = k_sweep_rows<512,1> + k_sweep_cols<512>",
+                     "kernel": "slice step = k_sweep_rows<512,1> + k_tile_cols<512>",
                      "launches": "eager, one stream, %d probes per launch (HIP events per launch)" % G,
                      "bytes_per_probe_slice": bytes_per_probe_slice},
     }

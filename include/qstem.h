@@ -300,11 +300,11 @@ int qs_adjoint_saved(qs_ctx *ctx, float *grad_V, float *grad_probe);
 int qs_atom_gradients(qs_ctx *ctx, const qs_atom *atoms, int natom, const qs_pot_params *pp, float *grad_xyz);
 
 /* Probes advanced together through all slices before the next group starts
- * (0 = library default).  batch = 1 is the per-probe launch sequence.  With the
- * default, qs_run_stem and qs_run_slices take windows of 64 and 128 points per side
- * through all slices in one launch (at 128 x 128 from 24 probes; not under
- * qs_set_profiling); a probe's results on the two sides of that line, and with a set
- * group size, agree to FP32 rounding. */
+ * (0 = library default).  batch = 1 is the per-probe launch sequence.  With any other
+ * value qs_run_stem and qs_run_slices take all probes of windows of 64 and 128 points
+ * per side through all slices in one launch (at 128 x 128 from 24 probes; not under
+ * qs_set_profiling); a probe's results on the two sides of that line, and with
+ * batch = 1, agree to FP32 rounding. */
 int qs_set_batch(qs_ctx *ctx, int batch);
 int qs_get_batch(const qs_ctx *ctx);
 

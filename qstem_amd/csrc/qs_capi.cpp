@@ -1431,14 +1431,14 @@ static void fill_sweep_args(qs_ctx* c, RunPlan& r, const int* d_ipos, const int*
   a.diff_scale = (float)pow((double)p.nx * p.ny, 1.5);
 }
 
-// Whether a qs_run_slices call is one launch of k_slab: windows that one CU holds, with the
-// library's group size (a set one, and per-launch profiling, keep the two sweeps).  20 slices,
+// Whether a qs_run_slices call is one launch of k_slab: windows that one CU holds (a group size
+// of 1, the per-probe launch sequence, and per-launch profiling keep the two sweeps).  20 slices,
 // sweeps / k_slab: of 64^2 one probe 220 / 162 us, 128 probes 310 / 166; of
 // 128 x 64 one 255 / 201; of 128^2, where a CU takes as long for a slice as the sweeps'
 // launches, 16 probes 274 / 296, 24 298 / 297, 128 566 / 307.
 static bool slab_run(const qs_ctx* c, int nprobe) {
   const qs_params& p = c->p;
-  return !c->generic && !c->profiling && c->batch == 0 && (nprobe >= 24 || p.nx * p.ny < 128 * 128) &&
+  return !c->generic && !c->profiling && c->batch != 1 && (nprobe >= 24 || p.nx * p.ny < 128 * 128) &&
          qs::slab_fits(p.nx, p.ny, c->kc);
 }
 
@@ -2674,7 +2674,7 @@ int qs_autotune(qs_ctx* c, const int* ipos, int nprobe, int* batch, int* rows_pe
         if (rc == QS_OK && (B <= n || B == Bs[0])) rc = consider(std::min(B, n), 0, 0);
     }
     const int B0 = best.batch;
-    if (c->batch == 0 && slab_run(c, n)) {
+    if (slab_run(c, n)) {
       // (one launch: the sweeps' shapes do not enter)
     } else if (c->mixed) {
       for (int rw : {1, 2, 4, 8, 16})

@@ -10,7 +10,8 @@
 // transformed.  The sweeps of qs_sweep.hpp take two dependent launches of 4.5 us (one probe of
 // 128^2) to 12 us (128 probes) each per slice; here a slice takes 12 us for up to 256 probes,
 // bounded by the CU's vector instructions and LDS accesses (about 9 us and 7 us of them).
-// A scan of 128 probes of 128^2 over 20 slices: 620 -> 296 us.
+// A scan of 256 probes of 128^2 over 20 slices: 630 -> 300 us (the rule of its use, with both
+// sides: slab_run in qs_capi.cpp).
 #include <hip/hip_runtime.h>
 
 #include "qs_sweep.hpp"

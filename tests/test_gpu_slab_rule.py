@@ -1,6 +1,6 @@
-"""Which kernels a small window's run takes: the one-launch kernel with the library's group
-size, the two sweeps (which per-launch profiling keeps too) with a set one; and the
-autotuner, which leaves the group size of such windows to the library."""
+"""Which kernels a small window's run takes: the one-launch kernel, or the two sweeps (which
+per-launch profiling keeps too) for the per-probe launch sequence of a group size of 1; and
+the autotuner, which leaves the group size of such windows to the library."""
 import numpy as np
 import pytest
 
@@ -23,9 +23,9 @@ def test_set_group_size_and_autotuner(nx, ny, probes):
         ms.set_profiling(False)
         one_launch = nx * ny < 128 * 128 or probes >= 24
         assert np.array_equal(whole, sweeps) == (not one_launch)
-        for batch in (1, 4):
+        for batch, want in ((1, sweeps), (4, whole)):
             ms.set_batch(batch)
-            assert np.array_equal(ms.run_stem(ipos, want_exit=True)["exit"], sweeps)
+            assert np.array_equal(ms.run_stem(ipos, want_exit=True)["exit"], want)
         ms.set_batch(0)
         best = ms.autotune(ipos)
         assert best["batch"] == 0 and ms.get_tuning()[2] == 0 and best["rate"] > 0
