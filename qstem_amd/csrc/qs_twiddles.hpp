@@ -24,12 +24,15 @@ std::vector<F2> twiddles(int n) {
 // cosine is zero it is 2^-28 and the tangent 2^28, off by 4e-9 of phase.
 //
 // Rounded with the modulus kept: of the nine neighbouring pairs of floats, the one whose
-// squared error along the value, weighted 10 to 1 against the error across it, is least.  A
+// squared error along the value, weighted 30 to 1 against the error across it, is least.  A
 // modulus error is a gain that every transform applies again, and the sum over the slices of
 // a run was the largest error of its detector sums: with (cos, sin) rounded to nearest a
 // 512-point transform loses 2.5e-8 of the amplitude, a 4096-point one 3.9e-8; so rounded
-// 1.1e-8 and 3e-9.  (Weights 3, 10, 100: gain at 4096 6, 3, 6e-9; rms error at 512 0.98, 0.99,
-// 1.00 of that of nearest pairs; dL/dV of probes of 256^2 5.0, 4.7, 4.9e-6.)
+// 1.3e-8 and 6e-9.  The weight is the one whose results were nearest to 64-bit ones: weights
+// 10, 30 and 100 give rms errors of dL/dV of 24 images of various sizes of 4.0, 3.7 and
+// 4.8e-6, and mean errors of dL/d(df0) of four sets of 1024 probes of 256^2 of 7.6, 2.0 and
+// 1.6e-6.  The error of a 512-point transform of random data is 1.00 (weight 10) or 1.02 (30)
+// of that with separate products by the nearest (cos, sin) at most.
 template <class F2>
 std::vector<F2> butterfly_twiddles(int n) {
   // the k-th float after v (not zero)
@@ -53,7 +56,7 @@ std::vector<F2> butterfly_twiddles(int n) {
         const float p = step((float)c, i), q = step((float)(s / c), k);
         const double x = p, y = (double)p * q;
         const double along = 0.5 * (x * x + y * y - 1.0), across = x * s - y * c;
-        const double cost = 10.0 * along * along + across * across;
+        const double cost = 30.0 * along * along + across * across;
         if (cost < best) {
           best = cost;
           t[m] = F2{p, q};
